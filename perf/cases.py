@@ -155,13 +155,14 @@ def _initial(case, n, seed):
     # the vortex carries 1e-3 of density noise; the others start smooth, as their resting states do
     noise = 2. * _random(cs, seed) - 1. if case["ic"] == "vortex" else 0. * one
     tp = 2. * math.pi
-    # a smooth three-dimensional flow and field under every kind; each face
-    # family's component depends on the transverse coordinates only, so the
-    # field starts free of divergence
+    # a smooth three-dimensional flow and field under the vortex and the blobs,
+    # rest and a uniform field under the blast; each face family's component
+    # depends on the transverse coordinates only, so the field starts free of
+    # divergence
     if case["ic"] == "vortex":
         amp, rho0, p0, b0, bu = 1., 25. / (36. * math.pi), 5. / (12. * math.pi), 1. / math.sqrt(4. * math.pi), .05
     elif case["ic"] == "blast":
-        amp, rho0, p0, b0, bu = .05, 1., .1, .05, .6
+        amp, rho0, p0, b0, bu = 0., 1., .1, 0., .6
     else:
         amp, rho0, p0, b0, bu = .2, 1., 1., .05, .29
     st = dict(rho=rho0 * (1. + 1e-3 * noise), p=p0 * one,
