@@ -1,4 +1,5 @@
-// Edge EMF (get_eijk_LFM, mhd3d3.f90:1754-1856) as a marching kernel.
+// Edge EMF (get_eijk_LFM, mhd3d3.f90:1754-1856) as a marching kernel (the
+// binary64 WENO reconstructions: mhd_emf_weno.hpp).
 //
 // Lanes run along x (every tap a coalesced load); each thread walks T edges
 // along a transverse axis and keeps the corner-velocity footprint of the

@@ -153,6 +153,13 @@ int mhd_create(mhd_ctx** out, const mhd_params* p) {
         plan.push_back({&c->flux[a], align_up(8 * c->nf[a] * tf)});
         plan.push_back({&c->emf[a], align_up(c->ne[a] * tf)});
     }
+    if ((p->reconop == 3 || p->reconop == 4) && p->precision == MHD_FP64) {
+        const size_t plane = 18 * (size_t)d.nx * d.ny * sizeof(double);
+        const long held = (long)(kWenoScratch / plane);
+        const long least = 16 + kWenoHalo, most = d.nz0 + 1 + kWenoHalo;
+        c->weno_planes = (int)std::min(most, std::max(least, held));
+        plan.push_back({&c->weno, align_up(plane * c->weno_planes)});
+    }
     plan.push_back({(void**)&c->dtpart, align_up(c->ndtpart * sizeof(double))});
     plan.push_back({(void**)&c->divpart, align_up(blocks(c->ninterior).x * sizeof(double))});
     plan.push_back({(void**)&c->scal, align_up(8 * sizeof(double))});

@@ -52,6 +52,12 @@ constexpr long kEmfFillThreads = 256L * 4 * 8 * 64;
 // default (mhd_set_stage_overlap)
 constexpr long kOverlapCells = 1L << 21;
 
+// scratch of the binary64 WENO EMF (mhd_emf_weno.hpp): 18 arrays over a
+// slab of whole planes, as many as kWenoScratch bytes hold (it should stay in
+// the last-level cache), at least kWenoHalo more than 16 planes of edges
+constexpr int kWenoHalo = 5;
+constexpr size_t kWenoScratch = size_t(160) << 20;
+
 struct mhd_ctx {
     mhd_params p{};
     mhd::Dims d{};
@@ -96,6 +102,8 @@ struct mhd_ctx {
     // per-stage products (binary64, or fp32 in mixed precision)
     void* flux[3] = {nullptr, nullptr, nullptr};
     void* emf[3] = {nullptr, nullptr, nullptr};
+    void* weno = nullptr;    // binary64 WENO contexts: the EMF's reconstructed lines, weno_planes planes of 18 arrays
+    int weno_planes = 0;
     double* dtpart = nullptr;
     double* divpart = nullptr;   // per-workgroup partials of the div B monitor (apart from the CFL ones)
     double* scal = nullptr;

@@ -4,6 +4,7 @@
 // parity), fp32 with FMA contraction (mixed precision).
 #pragma once
 #include "mhd_emf.hpp"
+#include "mhd_emf_weno.hpp"
 #include "mhd_launch.hpp"
 
 namespace mhd {
@@ -94,6 +95,33 @@ void emf_launch_k(mhd_ctx* c, EmfIn<TI> in) {
     else emf_launch_kt<R, M, K, EmfSteps<M, K>::T_SHORT, TI, TF>(c, in);
 }
 
+// the binary64 WENO reconstructions' EMF (mhd_emf_weno.hpp), slab by slab of z planes
+template <typename R, int M, typename TI, typename TF>
+void emf_weno_launch(mhd_ctx* c, const TI* const* u, Src<TI> s) {
+    const Dims& d = c->d;
+    const Coef<R> co = make_coef<R>(c);
+    EmfWenoIn<TI> in{{u[0], u[1], u[2]}, {s.bi, s.bj, s.bk}, s.vf, {}};
+    EmfWenoOut<R, TF> out{};
+    for (int a = 0; a < 3; ++a) {
+        out.e[a] = (TF*)c->emf[a];
+        out.ef[a] = R(c->met.ef[a]);
+        in.efa[a] = c->met.mode == 2 ? c->gm.ef[a] : nullptr;
+    }
+    const long plane = (long)d.nx * d.ny;
+    const int per = c->weno_planes - kWenoHalo;   // edge planes a slab holds
+    for (int k0 = 1; k0 <= d.nz0 + 1; k0 += per) {
+        const int k1 = k0 + per - 1 < d.nz0 + 1 ? k0 + per - 1 : d.nz0 + 1;
+        const WenoLines<R> ln{(R*)c->weno, plane * c->weno_planes, d.ng + k0 - 3};
+        const long nl = plane * (k1 - k0 + 1 + kWenoHalo);
+        launch(c, MHD_K_EMF, dim3(blocks(nl).x, 9), dim3(kBlock), k_weno_lines<R, M, TI>, d, co, u[0], u[1], u[2], ln,
+               k0, k1, nl);
+        // the most edges of the three directions in the slab
+        const long nm = (long)(d.nx0 + 1) * (d.ny0 + 1) * (k1 - k0 + 1);
+        launch(c, MHD_K_EMF, dim3(blocks(nm).x, 3), dim3(kBlock), k_emf_weno<R, M, TI, TF>, d, co, in, out, ln, k0,
+               k1);
+    }
+}
+
 // edge k: (v1, v2, b1, b2) = (vy, vz, bj, bk), (vz, vx, bk, bi), (vx, vy, bi, bj);
 // with a metric the velocities are the face-normal ones w_d = v . n_d
 template <typename R, typename TI, typename TF, int M>
@@ -104,9 +132,17 @@ void emf_launch_m(mhd_ctx* c, Src<TI> s) {
         u[1] = s.w[1];
         u[2] = s.w[2];
     }
-    emf_launch_k<R, M, 1, TI, TF>(c, EmfIn<TI>{u[1], u[2], s.bj, s.bk, s.vf});
-    emf_launch_k<R, M, 2, TI, TF>(c, EmfIn<TI>{u[2], u[0], s.bk, s.bi, s.vf});
-    emf_launch_k<R, M, 3, TI, TF>(c, EmfIn<TI>{u[0], u[1], s.bi, s.bj, s.vf});
+    // in binary64 the WENO footprint's lines are reconstructed once for all the
+    // edges they serve; in fp32 the march stays: which products of a line its
+    // compiler contracts depends on the line's place in the footprint, so
+    // shared lines would round differently by up to 2e-7 of an edge's EMF
+    if constexpr ((M == WENO5 || M == MPWENO5) && sizeof(R) == 8) {
+        emf_weno_launch<R, M, TI, TF>(c, u, s);
+    } else {
+        emf_launch_k<R, M, 1, TI, TF>(c, EmfIn<TI>{u[1], u[2], s.bj, s.bk, s.vf});
+        emf_launch_k<R, M, 2, TI, TF>(c, EmfIn<TI>{u[2], u[0], s.bk, s.bi, s.vf});
+        emf_launch_k<R, M, 3, TI, TF>(c, EmfIn<TI>{u[0], u[1], s.bi, s.bj, s.vf});
+    }
 }
 
 template <typename R, typename TI, typename TF>
