@@ -17,7 +17,7 @@
 // wavefronts per SIMD).  Both kernels are bound by VALU issue (the divisions
 // of the WENO weights): the states' round trip through memory is 18 words per
 // cell.  All three directions of the 96 x 64 x 128 shell (WENO5) took 1154 us
-// with that kernel and take 443 us (lines 118 us, edges 325 us) with these.
+// with that kernel and take 363 us with these (lines 95 us, edges 268 us).
 // The operations of each reconstruction, and so the results, are the
 // reference's bit for bit.
 //

@@ -153,13 +153,6 @@ int mhd_create(mhd_ctx** out, const mhd_params* p) {
         plan.push_back({&c->flux[a], align_up(8 * c->nf[a] * tf)});
         plan.push_back({&c->emf[a], align_up(c->ne[a] * tf)});
     }
-    if ((p->reconop == 3 || p->reconop == 4) && p->precision == MHD_FP64) {
-        const size_t plane = 18 * (size_t)d.nx * d.ny * sizeof(double);
-        const long held = (long)(kWenoScratch / plane);
-        const long least = 16 + kWenoHalo, most = d.nz0 + 1 + kWenoHalo;
-        c->weno_planes = (int)std::min(most, std::max(least, held));
-        plan.push_back({&c->weno, align_up(plane * c->weno_planes)});
-    }
     plan.push_back({(void**)&c->dtpart, align_up(c->ndtpart * sizeof(double))});
     plan.push_back({(void**)&c->divpart, align_up(blocks(c->ninterior).x * sizeof(double))});
     plan.push_back({(void**)&c->scal, align_up(8 * sizeof(double))});
@@ -186,7 +179,16 @@ int mhd_create(mhd_ctx** out, const mhd_params* p) {
         plan.push_back({(void**)&c->bjp, align_up(c->nbj * sizeof(double))});
         plan.push_back({(void**)&c->bkp, align_up(c->nbk * sizeof(double))});
     }
-    size_t total = 0;
+    size_t total = 0, state = 0;
+    for (auto& e : plan) state += e.second;
+    // the EMF's scratch comes last and is not cleared: each launch writes what it reads
+    if ((p->reconop == 3 || p->reconop == 4) && p->precision == MHD_FP64) {
+        const size_t plane = 18 * (size_t)d.nx * d.ny * sizeof(double);
+        const long held = (long)(kWenoScratch / plane);
+        const long least = 16 + kWenoHalo, most = d.nz0 + 1 + kWenoHalo;
+        c->weno_planes = (int)std::min(most, std::max(least, held));
+        plan.push_back({&c->weno, align_up(plane * c->weno_planes)});
+    }
     for (auto& e : plan) total += e.second;
     if (hipMalloc(&c->arena, total) != hipSuccess) {
         delete c;
@@ -211,7 +213,7 @@ int mhd_create(mhd_ctx** out, const mhd_params* p) {
         return MHD_ERR_HIP;
     }
     // zero everything once so ghost shells and unused slots hold defined values
-    if (hipMemsetAsync(c->arena, 0, total, c->s) != hipSuccess || hipStreamSynchronize(c->s) != hipSuccess) {
+    if (hipMemsetAsync(c->arena, 0, state, c->s) != hipSuccess || hipStreamSynchronize(c->s) != hipSuccess) {
         mhd_destroy(c);
         return MHD_ERR_HIP;
     }
