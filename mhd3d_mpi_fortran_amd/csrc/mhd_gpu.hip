@@ -135,7 +135,9 @@ int mhd_create(mhd_ctx** out, const mhd_params* p) {
     nmax = c->nbj > nmax ? c->nbj : nmax;
     nmax = c->nbk > nmax ? c->nbk : nmax;
     c->nmax = nmax;
-    c->ndtpart = (nmax + kBlock - 1) / kBlock;
+    // k_bxyz's grid: the cells and the upper boundary faces
+    c->nbxyz = c->ncell + (long)d.ny * d.nz + (long)d.nx * d.nz + (long)d.nx * d.ny;
+    c->ndtpart = blocks(c->nbxyz).x;
     const size_t tf = p->precision == MHD_MIXED ? sizeof(float) : sizeof(double);
 
     // arena layout
@@ -700,6 +702,10 @@ static double** state_slot(mhd_ctx* c, int a) {
     return t[a];
 }
 
+static BcSet bc_set(const mhd_ctx* c) {
+    return BcSet{{c->d.nx0, c->d.ny0, c->d.nz0}, {c->p.bc[0], c->p.bc[1], c->p.bc[2]}};
+}
+
 static void do_fill(mhd_ctx* c) {
     FillSet fs;
     const Dims& d = c->d;
@@ -719,18 +725,16 @@ static void do_fill(mhd_ctx* c) {
         most = cnt > most ? cnt : most;
     }
     fs.narr = 8;
-    fs.n0[0] = d.nx0;
-    fs.n0[1] = d.ny0;
-    fs.n0[2] = d.nz0;
-    for (int a = 0; a < 3; ++a) fs.bc[a] = c->p.bc[a];
+    fs.b = bc_set(c);
     dim3 grid((unsigned)((most + kBlock - 1) / kBlock), 8);
     launch(c, MHD_K_FILL, grid, dim3(kBlock), k_fill, fs, d.ng);
     c->dt_fresh = false;
 }
 
-// get_bxyz on the current state, plus (optionally) vf, the fp32 stencil
-// copies and the CFL partials of the next get_dt
-static void do_bxyz(mhd_ctx* c, bool want_vf, bool want_shadow, bool want_dt, bool store_cellb = true) {
+// get_bxyz on the current state, plus (optionally) the ghost fill before it,
+// vf, the fp32 stencil copies and the CFL partials of the next get_dt
+static void do_bxyz(mhd_ctx* c, bool want_vf, bool want_shadow, bool want_dt, bool store_cellb = true,
+                    bool fill = false) {
     Shadow sh{};
     if (want_shadow && mixed(c))
         sh = Shadow{c->sh[0], c->sh[1], c->sh[2], c->sh[3], c->sh[4],  c->sh[5],
@@ -738,39 +742,35 @@ static void do_bxyz(mhd_ctx* c, bool want_vf, bool want_shadow, bool want_dt, bo
     // face-normal velocities where the EMF will read them: binary64 with vf,
     // fp32 with the stencil copies
     const BMet m = bmet(c, want_vf && !mixed(c), want_shadow && mixed(c));
-    auto kb = c->met.mode == 2 ? k_bxyz<true> : k_bxyz<false>;
-    launch(c, MHD_K_BXYZ, blocks(c->nmax), dim3(kBlock), kb, c->d, c->p.gam, c->p.cfl,
-           CFaces{c->bi, c->bj, c->bk}, CCells{c->rho, c->vx, c->vy, c->vz, c->pr},
-           store_cellb ? c->bx : (double*)nullptr, c->by, c->bz, want_vf ? c->vf : (double*)nullptr, sh, m,
-           sdx(c), sdy(c), sdz(c), want_dt ? c->dtpart : (double*)nullptr, c->ncell, c->nbi, c->nbj, c->nbk);
+    auto kb = c->met.mode == 2 ? (fill ? k_bxyz<true, true> : k_bxyz<true, false>)
+                               : (fill ? k_bxyz<false, true> : k_bxyz<false, false>);
+    const dim3 grid = blocks(fill || sh.rho ? c->nbxyz : c->ncell);
+    launch(c, MHD_K_BXYZ, grid, dim3(kBlock), kb, c->d, c->p.gam, c->p.cfl, Faces{c->bi, c->bj, c->bk},
+           Cells{c->rho, c->vx, c->vy, c->vz, c->pr}, bc_set(c), store_cellb ? c->bx : (double*)nullptr, c->by, c->bz,
+           want_vf ? c->vf : (double*)nullptr, sh, m, sdx(c), sdy(c), sdz(c),
+           want_dt ? c->dtpart : (double*)nullptr, c->ncell);
     c->dt_fresh = want_dt;
-    c->ndt_valid = blocks(c->nmax).x;
+    c->ndt_valid = grid.x;
     c->cellb_stale = !store_cellb;
     // mixed precision keeps the extrapolated state in the fp32 copies
     if (want_shadow && mixed(c)) c->pred_valid = false;
 }
 
 // get_dt on the current state; the minimum lands in scal[SC_DTCFL] and, when
-// set_tau, also in scal[SC_TAU] (Adams-Bashforth takes tau from the CFL)
-static void do_dt(mhd_ctx* c, bool set_tau) {
+// set_tau, also in scal[SC_TAU] (Adams-Bashforth takes tau from the CFL);
+// fixed != null: tau = tau0 = *fixed instead (Runge-Kutta)
+static void do_dt(mhd_ctx* c, bool set_tau, const double* fixed = nullptr) {
     // where cell B of the current state is not stored (mixed Adams-Bashforth
     // steps, uploads), get_bxyz forms it and the CFL partials in one pass
     if (!c->dt_fresh && c->cellb_stale) do_bxyz(c, false, false, true);
+    long n = c->ndt_valid;
     if (!c->dt_fresh) {
         launch(c, MHD_K_DT, blocks(c->ncell), dim3(kBlock), k_dt_partial, c->d, c->p.gam, c->p.cfl, cur_state(c),
                sdx(c), sdy(c), sdz(c), gmet(c), c->dtpart, c->ncell);
-        launch(c, MHD_K_DT, dim3(1), dim3(1024), k_dt_final, (const double*)c->dtpart, blocks(c->ncell).x * 1L,
-               c->scal + SC_DTCFL, set_tau ? c->scal + SC_TAU : (double*)nullptr);
-        return;
+        n = blocks(c->ncell).x;
     }
-    launch(c, MHD_K_DT, dim3(1), dim3(1024), k_dt_final, (const double*)c->dtpart, c->ndt_valid, c->scal + SC_DTCFL,
-           set_tau ? c->scal + SC_TAU : (double*)nullptr);
-}
-
-static void do_prev_rk(mhd_ctx* c) {
-    launch(c, MHD_K_PREV, blocks(c->nmax), dim3(kBlock), k_prev_rk, c->p.gam - 1., cur_state(c), c->rhop, c->mxp,
-           c->myp, c->mzp, c->engp, (const double*)c->bi, (const double*)c->bj, (const double*)c->bk, c->bip,
-           c->bjp, c->bkp, c->ncell, c->nbi, c->nbj, c->nbk);
+    launch(c, MHD_K_DT, dim3(1), dim3(1024), k_dt_final, (const double*)c->dtpart, n, c->scal + SC_DTCFL,
+           set_tau || fixed ? c->scal + SC_TAU : (double*)nullptr, fixed ? 1 : 0, fixed ? *fixed : 0.);
 }
 
 // conserved update from the current state into `out` (the current state
@@ -809,7 +809,7 @@ template <typename TF, int NST, int ST>
 static void do_ct_t(mhd_ctx* c, double* const* out) {
     CFaces b{c->bi, c->bj, c->bk};
     Faces bo{out[8], out[9], out[10]};
-    CFaces bp{c->bip, c->bjp, c->bkp};
+    Faces bp{c->bip, c->bjp, c->bkp};
     const long nct = (long)(c->d.nx0 + 1) * c->d.ny0 * c->d.nz0 + (long)c->d.nx0 * (c->d.ny0 + 1) * c->d.nz0 +
                      (long)c->d.nx0 * c->d.ny0 * (c->d.nz0 + 1);
     const CtFactor ctf{{c->met.ct[0], c->met.ct[1], c->met.ct[2]}};
@@ -1104,11 +1104,13 @@ int mhd_flux_stress_old(mhd_ctx* c) { return mhd_flux_stress(c, MHD_STATE_PREDIC
 // vf and fp32 copies are kept only where the next step reads them: RK reads
 // the current state (vf in binary64, the copies in mixed precision), AB
 // reads the extrapolated state written by the predictor
-static void end_of_stage(mhd_ctx* c, bool in_step = false) {
+// The ghost fill rides along; `last`: the CFL partials, which only the next
+// step reads, are wanted
+static void end_of_stage(mhd_ctx* c, bool in_step = false, bool last = true) {
     const bool rk = c->p.stepop != 1;
     // mixed Adams-Bashforth steps take the extrapolated cell B from the faces
     // (k_predict_ab_mixed), so the step itself leaves cell B implicit
-    do_bxyz(c, rk && !mixed(c), rk && mixed(c), true, !(in_step && !rk && mixed(c)));
+    do_bxyz(c, rk && !mixed(c), rk && mixed(c), last, !(in_step && !rk && mixed(c)), true);
 }
 // cell B of the current state where a caller reads it
 static void ensure_cellb(mhd_ctx* c) {
@@ -1122,7 +1124,6 @@ int mhd_initialize(mhd_ctx* c, double* tau) {
     c->tau0_host = t;
     c->pred_valid = false;
     launch(c, MHD_K_PREV, dim3(1), dim3(64), k_set2, c->scal + SC_TAU, t, t);
-    do_fill(c);
     end_of_stage(c);
     double out = t;
     if (c->p.stepop == 1) {
@@ -1144,17 +1145,14 @@ int mhd_initialize(mhd_ctx* c, double* tau) {
 // step_rk2 / step_rk3 (mhd3d3.f90:3648-3792), in place
 template <int NST>
 static void step_rk(mhd_ctx* c) {
-    do_dt(c, false);
-    launch(c, MHD_K_PREV, dim3(1), dim3(64), k_set2, c->scal + SC_TAU, c->tau0_host, c->tau0_host);
-    do_prev_rk(c);
+    do_dt(c, false, &c->tau0_host);
     double* self[11];
     for (int a = 0; a < 11; ++a) self[a] = *state_slot(c, a);
     for (int st = 1; st <= NST; ++st) {
         if (st == 1) do_stage<NST, 1>(c, cur_src(c), self);
         else if (st == 2) do_stage<NST, 2>(c, cur_src(c), self);
         else do_stage<NST, 3>(c, cur_src(c), self);
-        do_fill(c);
-        end_of_stage(c);
+        end_of_stage(c, true, st == NST);
     }
 }
 
@@ -1209,8 +1207,8 @@ static void step_ab(mhd_ctx* c) {
         c->xn[a] = c->xp[a];
         c->xp[a] = cur;
     }
-    do_fill(c);
     if (fuse_dt(c)) {  // the update left the CFL partials of the new state
+        do_fill(c);
         c->dt_fresh = true;
         c->ndt_valid = fused ? fused_blocks(c->d) : blocks(c->ninterior).x;
         c->cellb_stale = true;
@@ -1299,7 +1297,6 @@ int mhd_advance(mhd_ctx* c, int stage) {
     const int nst = c->p.stepop == 1 ? 0 : c->p.stepop;
     if (nst == 0 ? stage != 0 : (stage < 1 || stage > nst)) return MHD_ERR_PARAM;
     hipSetDevice(c->p.device);
-    if (stage == 1) do_prev_rk(c);   // advance_previous: the state stage 1 starts from
     if (nst == 0) advance_serial<0, 0>(c);
     else if (nst == 2 && stage == 1) advance_serial<2, 1>(c);
     else if (nst == 2) advance_serial<2, 2>(c);
@@ -1576,7 +1573,7 @@ int mhd_divb_max(mhd_ctx* c, double* divb) {
     launch(c, MHD_K_DT, g, dim3(kBlock), k, c->d, CFaces{c->bi, c->bj, c->bk}, sdx(c), sdy(c), sdz(c), gmet(c),
            c->divpart, c->ninterior);
     launch(c, MHD_K_DT, dim3(1), dim3(1024), k_dt_final, (const double*)c->divpart, (long)g.x, c->scal + SC_DIVB,
-           (double*)nullptr);
+           (double*)nullptr, 0, 0.);
     double h = 0.;
     if (hipMemcpyAsync(&h, c->scal + SC_DIVB, sizeof(double), hipMemcpyDeviceToHost, c->s) != hipSuccess)
         return MHD_ERR_HIP;

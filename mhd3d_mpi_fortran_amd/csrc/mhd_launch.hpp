@@ -72,7 +72,7 @@ struct mhd_ctx {
     char* arena = nullptr;
     size_t arena_bytes = 0;
     bool have_geometry = false;
-    long ncell = 0, nbi = 0, nbj = 0, nbk = 0, ninterior = 0, ndtpart = 0, nmax = 0;
+    long ncell = 0, nbi = 0, nbj = 0, nbk = 0, ninterior = 0, ndtpart = 0, nbxyz = 0, nmax = 0;
     long nf[3] = {0, 0, 0}, ne[3] = {0, 0, 0};
     // EMF launches with fewer long-run threads than this take short runs
     // (environment MHD_EMF_FILL_THREADS overrides it at mhd_create)

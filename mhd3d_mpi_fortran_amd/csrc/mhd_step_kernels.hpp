@@ -13,6 +13,10 @@ namespace mhd {
 // (mhd3d3.f90:1641-1650, 3842-3907, 3648-3792).
 //   NST = 0: Adams-Bashforth corrector (no combine, p from the new momentum)
 //   NST = 2/3: TVD RK stage ST
+// A Runge-Kutta stage 1 holds advance_previous' copies (the conserved state it
+// starts from, mhd3d3.f90:3794-3819) in registers and stores them for the
+// later stages, which saves the pass that read the state again (k_ct does
+// the same for the faces): at 96^3 that pass took 26 us a step.
 // ------------------------------------------------------------------------
 struct Cells {  // cell primitives written by the update
     double *rho, *vx, *vy, *vz, *p;
@@ -20,8 +24,8 @@ struct Cells {  // cell primitives written by the update
 struct CCells {  // cell primitives the update starts from
     const double *rho, *vx, *vy, *vz, *p;
 };
-struct PrevRK {  // advance_previous, RK flavour
-    const double *rho, *mx, *my, *mz, *eng;
+struct PrevRK {  // advance_previous, RK flavour (owned cells)
+    double *rho, *mx, *my, *mz, *eng;
 };
 
 template <typename TF>
@@ -100,7 +104,13 @@ __global__ void __launch_bounds__(kBlock) k_update(Dims d, double gm1, const dou
     double my = my0 - tau * div(2);
     double mz = mz0 - tau * div(3);
     double hx = mx, hy = my, hz = mz;
-    if (NST == 2 && ST == 2) {
+    if (NST > 0 && ST == 1) {
+        pv.rho[q] = r0;
+        pv.mx[q] = mx0;
+        pv.my[q] = my0;
+        pv.mz[q] = mz0;
+        pv.eng[q] = e0;
+    } else if (NST == 2 && ST == 2) {
         rho = (pv.rho[q] + rho) / 2.;
         hx = (pv.mx[q] + mx) / 2.;
         hy = (pv.my[q] + my) / 2.;
@@ -187,7 +197,7 @@ struct CtFactor {
 // by the face's area
 template <int NST, int ST, typename TF, bool GEN>
 __global__ void __launch_bounds__(kBlock) k_ct(Dims d, const double* __restrict__ tau_p, CtFactor ctf, CFaces b,
-                                              Faces bo, CFaces bp, const TF* __restrict__ ei,
+                                              Faces bo, Faces bp, const TF* __restrict__ ei,
                                               const TF* __restrict__ ej, const TF* __restrict__ ek,
                                               const double* __restrict__ dx, const double* __restrict__ dy,
                                               const double* __restrict__ dz, GMet gm) {
@@ -200,8 +210,7 @@ __global__ void __launch_bounds__(kBlock) k_ct(Dims d, const double* __restrict_
     int i, j, k;
     double val, old;
     ptrdiff_t q;
-    double* out;
-    const double* prev;
+    double *out, *prev;
     if (t < nbi) {
         unflat(t, nx0 + 1, ny0, i, j, k);
         // ek (nx0+1,ny0+1,nz0), ej (nx0+1,ny0,nz0+1)
@@ -239,8 +248,8 @@ __global__ void __launch_bounds__(kBlock) k_ct(Dims d, const double* __restrict_
         out = bo.bk;
         prev = bp.bk;
     }
-    (void)old;
-    if (NST == 2 && ST == 2) val = (prev[q] + val) / 2.;
+    if (NST > 0 && ST == 1) prev[q] = old;
+    else if (NST == 2 && ST == 2) val = (prev[q] + val) / 2.;
     else if (NST == 3 && ST == 2) val = (3. * prev[q] + val) / 4.;
     else if (NST == 3 && ST == 3) val = (prev[q] + 2. * val) / 3.;
     out[q] = val;
@@ -258,11 +267,14 @@ struct FillArr {
     int n[3];     // extents
     int face;     // 0 cells, 1..3 normal axis of a face array
 };
+struct BcSet {
+    int n0[3];
+    int bc[3];    // 0 even reflection, 2 periodic
+};
 struct FillSet {
     FillArr arr[8];
     int narr;
-    int n0[3];
-    int bc[3];    // 0 even reflection, 2 periodic
+    BcSet b;
 };
 
 __device__ __forceinline__ int fill_map(int i, int n0, int ng, bool face, int bc) {
@@ -281,7 +293,7 @@ __global__ void __launch_bounds__(kBlock) k_fill(FillSet fs, int ng) {
 #pragma unroll
     for (int a = 0; a < 3; ++a) {
         len[a] = A.n[a];
-        own[a] = fs.n0[a] + (A.face == a + 1 ? 1 : 0);
+        own[a] = fs.b.n0[a] + (A.face == a + 1 ? 1 : 0);
     }
     const int g2 = 2 * ng;
     const long c1 = (long)g2 * len[1] * len[2];
@@ -308,19 +320,28 @@ __global__ void __launch_bounds__(kBlock) k_fill(FillSet fs, int ng) {
     } else {
         return;
     }
-    const int si = fill_map(i, fs.n0[0], ng, A.face == 1, fs.bc[0]);
-    const int sj = fill_map(j, fs.n0[1], ng, A.face == 2, fs.bc[1]);
-    const int sk = fill_map(k, fs.n0[2], ng, A.face == 3, fs.bc[2]);
+    const int si = fill_map(i, fs.b.n0[0], ng, A.face == 1, fs.b.bc[0]);
+    const int sj = fill_map(j, fs.b.n0[1], ng, A.face == 2, fs.b.bc[1]);
+    const int sk = fill_map(k, fs.b.n0[2], ng, A.face == 3, fs.b.bc[2]);
     A.a[ix(len[0], len[1], i, j, k)] = A.a[ix(len[0], len[1], si, sj, sk)];
 }
 
 // ------------------------------------------------------------------------
 // get_bxyz (mhd3d3.f90:2118-2128) over the ghost-inclusive block, fused with
+//   * the ghost fill (FILL): a ghost cell or face takes its value from the
+//     owned one that k_fill copies it from, and stores it -- every read is of
+//     an owned element, every ghost write of this thread's own, so no thread
+//     reads what another writes.  The pass reads what k_fill wrote, so
+//     folding it in costs index arithmetic only (16^3: 4.4 us a stage for the
+//     two kernels' 7.5; a 64^3 PDM RK2 step with the other passes saved here
+//     317 -> 298 us),
 //   * the EMF's fast speed vf=|v|+|B|/sqrt(rho) (mhd3d3.f90:1766) when vf != 0,
 //   * fp32 copies of the stencil inputs (mixed precision) when sh.rho != 0,
 //   * per-workgroup minima of the CFL dt (get_dt, mhd3d3.f90:1608-1628)
 //     when part != 0 -- the dt the next step starts with.
-// Threads cover max(ncell, nbi, nbj, nbk) so the face copies ride along.
+// Threads: one per cell, which also does the cell's lower faces, then one per
+// face that is no cell's lower face (i = nx+1 of bi, j = ny+1 of bj, k = nz+1
+// of bk; left out when neither FILL nor the copies need them).
 // ------------------------------------------------------------------------
 struct Shadow {  // fp32 stencil inputs of one state
     float *rho, *vx, *vy, *vz, *p, *bx, *by, *bz, *vf, *bi, *bj, *bk;
@@ -360,25 +381,49 @@ __device__ __forceinline__ double cfl_dt_gen(double gam, double cfl, double u, d
 }
 
 // GEN: general metric (met.g)
-template <bool GEN>
-__global__ void __launch_bounds__(kBlock) k_bxyz(Dims d, double gam, double cfl, CFaces b, CCells s,
+template <bool GEN, bool FILL>
+__global__ void __launch_bounds__(kBlock) k_bxyz(Dims d, double gam, double cfl, Faces b, Cells s, BcSet bc,
                                                 double* __restrict__ bx, double* __restrict__ by,
                                                 double* __restrict__ bz, double* __restrict__ vf, Shadow sh, BMet met,
                                                 const double* __restrict__ dx, const double* __restrict__ dy,
-                                                const double* __restrict__ dz, double* __restrict__ part, long ncell,
-                                                long nbi, long nbj, long nbk) {
+                                                const double* __restrict__ dz, double* __restrict__ part, long ncell) {
     const long t = gtid_xcd();
+    const int ng = d.ng;
+    // the index an element's value comes from, per axis: cells and faces
+    auto cm = [&](int a, int i) { return FILL ? fill_map(i, bc.n0[a], ng, false, bc.bc[a]) : i; };
+    auto fm = [&](int a, int i) { return FILL ? fill_map(i, bc.n0[a], ng, true, bc.bc[a]) : i; };
     double dt = __builtin_huge_val();
     if (t < ncell) {
         int i, j, k;
         unflat(t, d.nx, d.ny, i, j, k);
-        const double bi0 = b.bi[ix(d.nx + 1, d.ny, i, j, k)], bi1 = b.bi[ix(d.nx + 1, d.ny, i + 1, j, k)];
-        const double bj0 = b.bj[ix(d.nx, d.ny + 1, i, j, k)], bj1 = b.bj[ix(d.nx, d.ny + 1, i, j + 1, k)];
-        const double bk0 = b.bk[t], bk1 = b.bk[t + (ptrdiff_t)d.nx * d.ny];
+        const int si = cm(0, i), sj = cm(1, j), sk = cm(2, k);
+        const int fi = fm(0, i), fj = fm(1, j), fk = fm(2, k);
+        const ptrdiff_t q = ix(d.nx, d.ny, si, sj, sk);
+        const double bi0 = b.bi[ix(d.nx + 1, d.ny, fi, sj, sk)], bi1 = b.bi[ix(d.nx + 1, d.ny, fm(0, i + 1), sj, sk)];
+        const double bj0 = b.bj[ix(d.nx, d.ny + 1, si, fj, sk)], bj1 = b.bj[ix(d.nx, d.ny + 1, si, fm(1, j + 1), sk)];
+        const double bk0 = b.bk[ix(d.nx, d.ny, si, sj, fk)], bk1 = b.bk[ix(d.nx, d.ny, si, sj, fm(2, k + 1))];
         double x = .5 * (bi1 + bi0);
         double y = .5 * (bj1 + bj0);
         double z = .5 * (bk1 + bk0);
-        const double u = s.vx[t], v = s.vy[t], w = s.vz[t], r = s.rho[t], pp = s.p[t];
+        const double u = s.vx[q], v = s.vy[q], w = s.vz[q], r = s.rho[q], pp = s.p[q];
+        if constexpr (FILL) {
+            const bool gx = si != i, gy = sj != j, gz = sk != k;
+            if (gx || gy || gz) {
+                s.rho[t] = r;
+                s.vx[t] = u;
+                s.vy[t] = v;
+                s.vz[t] = w;
+                s.p[t] = pp;
+            }
+            if (fi != i || gy || gz) b.bi[ix(d.nx + 1, d.ny, i, j, k)] = bi0;
+            if (gx || fj != j || gz) b.bj[ix(d.nx, d.ny + 1, i, j, k)] = bj0;
+            if (gx || gy || fk != k) b.bk[t] = bk0;
+        }
+        if (sh.rho) {
+            sh.bi[ix(d.nx + 1, d.ny, i, j, k)] = float(bi0);
+            sh.bj[ix(d.nx, d.ny + 1, i, j, k)] = float(bj0);
+            sh.bk[t] = float(bk0);
+        }
         if constexpr (GEN) {
             const double beta[6] = {bi0, bi1, bj0, bj1, bk0, bk1};
             double B[3];
@@ -429,11 +474,28 @@ __global__ void __launch_bounds__(kBlock) k_bxyz(Dims d, double gam, double cfl,
         if (part)
             dt = GEN ? cfl_dt_gen(gam, cfl, u, v, w, x, y, z, r, pp, met.g, t)
                             : cfl_dt(gam, cfl, u, v, w, x, y, z, r, pp, dx[i - 1], dy[j - 1], dz[k - 1]);
-    }
-    if (sh.bi) {
-        if (t < nbi) sh.bi[t] = float(b.bi[t]);
-        if (t < nbj) sh.bj[t] = float(b.bj[t]);
-        if (t < nbk) sh.bk[t] = float(b.bk[t]);
+    } else {
+        long e = t - ncell;
+        const long nyz = (long)d.ny * d.nz, nxz = (long)d.nx * d.nz, nxy = (long)d.nx * d.ny;
+        if (e < nyz) {
+            const int j = (int)(e % d.ny) + 1, k = (int)(e / d.ny) + 1;
+            const ptrdiff_t f = ix(d.nx + 1, d.ny, d.nx + 1, j, k);
+            const double val = b.bi[ix(d.nx + 1, d.ny, fm(0, d.nx + 1), cm(1, j), cm(2, k))];
+            if (FILL) b.bi[f] = val;
+            if (sh.rho) sh.bi[f] = float(val);
+        } else if ((e -= nyz) < nxz) {
+            const int i = (int)(e % d.nx) + 1, k = (int)(e / d.nx) + 1;
+            const ptrdiff_t f = ix(d.nx, d.ny + 1, i, d.ny + 1, k);
+            const double val = b.bj[ix(d.nx, d.ny + 1, cm(0, i), fm(1, d.ny + 1), cm(2, k))];
+            if (FILL) b.bj[f] = val;
+            if (sh.rho) sh.bj[f] = float(val);
+        } else if ((e -= nxz) < nxy) {
+            const int i = (int)(e % d.nx) + 1, j = (int)(e / d.nx) + 1;
+            const ptrdiff_t f = ix(d.nx, d.ny, i, j, d.nz + 1);
+            const double val = b.bk[ix(d.nx, d.ny, cm(0, i), cm(1, j), fm(2, d.nz + 1))];
+            if (FILL) b.bk[f] = val;
+            if (sh.rho) sh.bk[f] = float(val);
+        }
     }
     if (part) {
         dt = block_min(dt);
@@ -472,7 +534,6 @@ __global__ void __launch_bounds__(kBlock) k_dt_partial(Dims d, double gam, doubl
     if (threadIdx.x == 0) part[blockIdx.x] = dt;
 }
 
-// out[0] = min(part); if tau != null also tau[0] = out[0] (AB: tau from CFL)
 // divergence monitor: -|div B| of each interior cell, as the update forms a
 // flux divergence (tensor or affine metric: differences over the metric
 // spacing; general metric: face fluxes times areas over the volume); the
@@ -506,8 +567,11 @@ __global__ void __launch_bounds__(kBlock) k_divb_partial(Dims d, CFaces b, const
     if (threadIdx.x == 0) part[blockIdx.x] = v;
 }
 
+// out[0] = min(part); Adams-Bashforth takes its step from it (tau != null:
+// tau[0] = out[0]), Runge-Kutta keeps its own (fixed: tau = tau0 = fix)
 __global__ void __launch_bounds__(1024) k_dt_final(const double* __restrict__ part, long npart,
-                                                   double* __restrict__ out, double* __restrict__ tau) {
+                                                   double* __restrict__ out, double* __restrict__ tau,
+                                                   int fixed, double fix) {
     __shared__ double red[16];
     // eight loads in flight per thread (one after the other, the 64 k partials
     // of a 256^3 block took 32 us); the minimum does not depend on the order
@@ -535,7 +599,12 @@ __global__ void __launch_bounds__(1024) k_dt_final(const double* __restrict__ pa
         double r = red[0];
         for (int q = 1; q < (int)(blockDim.x >> 6); ++q) r = red[q] < r ? red[q] : r;
         out[0] = r;
-        if (tau) tau[0] = r;
+        if (fixed) {
+            tau[0] = fix;
+            tau[1] = fix;
+        } else if (tau) {
+            tau[0] = r;
+        }
     }
 }
 
@@ -551,30 +620,6 @@ __global__ void k_zero_int(int* __restrict__ p) {
 }
 __global__ void k_tau0_from_tau(double* __restrict__ p) {
     if (threadIdx.x == 0 && blockIdx.x == 0) p[1] = p[0];
-}
-
-// ------------------------------------------------------------------------
-// advance_previous (mhd3d3.f90:3794-3819), RK flavour, full arrays
-// ------------------------------------------------------------------------
-__global__ void __launch_bounds__(kBlock) k_prev_rk(double gm1, Prim<double> q, double* __restrict__ rhop,
-                                                   double* __restrict__ mxp, double* __restrict__ myp,
-                                                   double* __restrict__ mzp, double* __restrict__ engp,
-                                                   const double* __restrict__ bi, const double* __restrict__ bj,
-                                                   const double* __restrict__ bk, double* __restrict__ bip,
-                                                   double* __restrict__ bjp, double* __restrict__ bkp, long ncell,
-                                                   long nbi, long nbj, long nbk) {
-    const long t = gtid();
-    if (t < ncell) {
-        const double r = q.rho[t], u = q.vx[t], v = q.vy[t], w = q.vz[t];
-        rhop[t] = r;
-        mxp[t] = r * u;
-        myp[t] = r * v;
-        mzp[t] = r * w;
-        engp[t] = .5 * r * (u * u + v * v + w * w) + q.p[t] / gm1;
-    }
-    if (t < nbi) bip[t] = bi[t];
-    if (t < nbj) bjp[t] = bj[t];
-    if (t < nbk) bkp[t] = bk[t];
 }
 
 // ------------------------------------------------------------------------
