@@ -406,199 +406,19 @@ template <typename R, int M, int K, int T, typename TI, typename TF>
 __global__ void __launch_bounds__(kBlock) k_emf_march(Dims d, Coef<R> c, EmfIn<TI> in, R ef,
                                                      const double* __restrict__ efa, TF* __restrict__ e,
                                                      long nthreads) {
-    const int ii = d.nx0 + (K != 1);
-    const int no = K == 3 ? d.nz0 : (K == 1 ? d.ny0 + 1 : d.ny0);
-    const int nm = K == 3 ? d.ny0 + 1 : d.nz0 + 1;
-    int i, o, mb;
-    if constexpr (K == 1) {
-        // both corner axes are strided for ei: a workgroup takes 64 x-lanes
-        // of 4 consecutive y edges (emf_tiles), whose four wavefronts share
-        // 11 of their 32 window rows per step in the CU's L1
-        const unsigned blk = xcd_block();
-        const unsigned ntx = (ii + kTileX - 1) / kTileX, nto = (no + kTileN - 1) / kTileN;
-        const unsigned tx = blk % ntx, r = blk / ntx, to = r % nto;
-        mb = (int)(r / nto);
-        i = (int)(tx * kTileX + (threadIdx.x & (kTileX - 1))) + 1;
-        o = (int)(to * kTileN + threadIdx.x / kTileX) + 1;
-        if (i > ii || o > no || (long)mb * T >= nm) return;
-    } else {
-        const long t = gtid_xcd();
-        if (t >= nthreads) return;
-        const unsigned r = (unsigned)t / (unsigned)ii;   // index spaces stay below 2^31
-        i = (int)((unsigned)t - r * (unsigned)ii) + 1;
-        mb = (int)(r / (unsigned)no);
-        o = (int)(r - (unsigned)mb * (unsigned)no) + 1;
-    }
-    // runs of exactly T edges: the last run of a line starts early; it
-    // stores only the edges that are its own (fp32 contraction may round an
-    // edge differently at another step of the run, and two threads writing
-    // one edge would leave whichever came last)
-    const int m0 = (mb * T < nm - T ? mb * T : nm - T) + 1;
-    const int skip = mb * T + 1 - m0;
-    // first edge of this thread
-    const int j0 = K == 3 ? m0 : o, k0 = K == 3 ? o : m0;
-    const int nx = d.nx, ny = d.ny, ng = d.ng;
-    const int I = ng + i, J = ng + j0, Kc = ng + k0;
-    const ptrdiff_t sx = 1, sy = nx, sz = (ptrdiff_t)nx * ny;
-    const ptrdiff_t s1 = K == 1 ? sy : (K == 2 ? sz : sx);
-    const ptrdiff_t s2 = K == 1 ? sz : (K == 2 ? sx : sy);
-    const ptrdiff_t smarch = K == 3 ? sy : sz;
-    const ptrdiff_t bc0 = ix(nx, ny, I, J, Kc);
-    constexpr bool MD1 = EmfGeom<K>::MD1;
+#define EMF_BLOCK() xcd_block()
+#include "mhd_emf_march.inc"
+#undef EMF_BLOCK
+}
 
-    // buffer views (array sizes in bytes): cell arrays and the two face arrays
-    constexpr unsigned E = sizeof(TI);
-    const unsigned ncell = (unsigned)nx * (unsigned)ny * (unsigned)d.nz;
-    const unsigned nf1 = K == 1 ? (unsigned)nx * (ny + 1) * d.nz : (K == 2 ? (unsigned)nx * ny * (d.nz + 1)
-                                                                           : (unsigned)(nx + 1) * ny * d.nz);
-    const unsigned nf2 = K == 1 ? (unsigned)nx * ny * (d.nz + 1) : (K == 2 ? (unsigned)(nx + 1) * ny * d.nz
-                                                                           : (unsigned)nx * (ny + 1) * d.nz);
-    const Buf<TI> bv1(in.v1, ncell * E), bv2(in.v2, ncell * E), bb1(in.b1, nf1 * E), bb2(in.b2, nf2 * E),
-        bvf(in.vf, ncell * E);
-
-    R v1av[T], v2av[T];
-    // the window's other axis is x (unit stride) for K=2 and K=3
-    if constexpr (M == PDM && !(MD1 && sizeof(R) == 8)) {
-        const ptrdiff_t sm = MD1 ? s1 : s2, so = MD1 ? s2 : s1;
-        const unsigned ob = (unsigned)bc0 * E, osm = (unsigned)sm * E, oso = (unsigned)so * E;
-        vav_march_pdm<R, MD1, K != 1, T>(in.v1, bv1, ob, osm, oso, c, v1av);
-        vav_march_pdm<R, MD1, K != 1, T>(in.v2, bv2, ob, osm, oso, c, v2av);
-    } else {
-        vav_march<R, M, MD1, K != 1, T>(in.v1, bc0, s1, s2, c, v1av);
-        vav_march<R, M, MD1, K != 1, T>(in.v2, bc0, s1, s2, c, v2av);
-    }
-
-    // face B reconstructions and the Alfven resistivity, edge by edge
-    ptrdiff_t base1, st1, base2, st2, mv1, mv2, ostr;
-    if (K == 1) {  // b1 = bj (nx,ny+1,nz) along z; b2 = bk (nx,ny,nz+1) along y; e (nx0,ny0+1,nz0+1)
-        base1 = ix(nx, ny + 1, I, J, Kc);
-        st1 = (ptrdiff_t)nx * (ny + 1);
-        mv1 = st1;
-        base2 = ix(nx, ny, I, J, Kc);
-        st2 = nx;
-        mv2 = (ptrdiff_t)nx * ny;
-        ostr = (ptrdiff_t)d.nx0 * (d.ny0 + 1);
-    } else if (K == 2) {  // b1 = bk along x; b2 = bi (nx+1,ny,nz) along z; e (nx0+1,ny0,nz0+1)
-        base1 = ix(nx, ny, I, J, Kc);
-        st1 = 1;
-        mv1 = (ptrdiff_t)nx * ny;
-        base2 = ix(nx + 1, ny, I, J, Kc);
-        st2 = (ptrdiff_t)(nx + 1) * ny;
-        mv2 = st2;
-        ostr = (ptrdiff_t)(d.nx0 + 1) * d.ny0;
-    } else {  // b1 = bi along y; b2 = bj along x; e (nx0+1,ny0+1,nz0)
-        base1 = ix(nx + 1, ny, I, J, Kc);
-        st1 = nx + 1;
-        mv1 = st1;
-        base2 = ix(nx, ny + 1, I, J, Kc);
-        st2 = 1;
-        mv2 = nx;
-        ostr = d.nx0 + 1;
-    }
-    ptrdiff_t eo = K == 1 ? ix(d.nx0, d.ny0 + 1, i, j0, k0)
-                          : (K == 2 ? ix(d.nx0 + 1, d.ny0, i, j0, k0) : ix(d.nx0 + 1, d.ny0 + 1, i, j0, k0));
-    // 32-bit byte offsets (every array stays below 2^32 bytes)
-    unsigned ob1 = (unsigned)base1 * E, ob2 = (unsigned)base2 * E, obc = (unsigned)bc0 * E;
-    const unsigned ost1 = (unsigned)st1 * E, ost2 = (unsigned)st2 * E, omv1 = (unsigned)mv1 * E,
-                   omv2 = (unsigned)mv2 * E, omarch = (unsigned)smarch * E;
-    const unsigned osx = E, osy = (unsigned)sy * E, osz = (unsigned)sz * E;
-    // One of the two face-B reconstructions runs along the march axis (b1 =
-    // bj along z for K=1, b2 = bi along z for K=2, b1 = bi along y for K=3):
-    // consecutive edges share all but one of its taps, which ride along in
-    // registers.  The other one's taps are contiguous (x: b1 for K=2, b2 for
-    // K=3) or strided (buffer loads with uniform offsets).  Of the four cells
-    // around the edge, two are the previous edge's.
-    using S = Stencil<R, M>;
-    constexpr bool MA1 = K != 2;
-    const Buf<TI>& bma = MA1 ? bb1 : bb2;
-    const unsigned ostma = MA1 ? ost1 : ost2;
-    R ta[S::n];
-    {
-        const unsigned o0 = (MA1 ? ob1 : ob2) + (unsigned)S::lo * ostma;
-#pragma unroll
-        for (int m = 0; m < S::n; ++m) ta[m] = R(bma.at(o0, (unsigned)m * ostma));
-    }
-    const unsigned ou = K == 1 ? osy : osx, ow = K == 3 ? osy : osz;
-    R f_uw = R(bvf.at(obc - ou - ow, 0u)), f_w = R(bvf.at(obc - ou - ow, ou));
-    // a step's loads: the taps of the reconstruction across the march, the
-    // march one's new tap and the two new cells; fp32 loads them one step
-    // ahead, so their latency hides behind the current step's arithmetic
-    struct StepTaps {
-        R o[S::n];
-        R nm, f0, fu;
-    };
-    auto load_taps = [&](unsigned o1s, unsigned o2s, unsigned ocs, StepTaps& t) {
-        if constexpr (K == 1) {
-            const unsigned o0 = o2s + (unsigned)S::lo * ost2;
-#pragma unroll
-            for (int m = 0; m < S::n; ++m) t.o[m] = R(bb2.at(o0, (unsigned)m * ost2));
-        } else {
-            const TI* q = reinterpret_cast<const TI*>(reinterpret_cast<const char*>(K == 2 ? in.b1 : in.b2) +
-                                                      (K == 2 ? o1s : o2s));
-#pragma unroll
-            for (int m = 0; m < S::n; ++m) t.o[m] = R(q[S::lo + m]);
-        }
-        t.nm = R(bma.at((MA1 ? o1s : o2s) + (unsigned)(S::lo + S::n - 1) * ostma, 0u));
-        t.f0 = R(bvf.at(ocs, 0u));
-        t.fu = R(bvf.at(ocs - ou, 0u));
-    };
-    constexpr bool PREB = sizeof(R) == 4;
-    StepTaps cur;
-    load_taps(ob1, ob2, obc, cur);
-#pragma unroll
-    for (int s = 0; s < T; ++s) {
-        {
-            StepTaps nxt;
-            if constexpr (PREB) {
-                if (s + 1 < T) load_taps(ob1 + omv1, ob2 + omv2, obc + omarch, nxt);
-            }
-            if (s > 0) {
-#pragma unroll
-                for (int m = 0; m < S::n - 1; ++m) ta[m] = ta[m + 1];
-                ta[S::n - 1] = cur.nm;
-            }
-            const R sig1 = sgn1(v1av[s]), sig2 = sgn1(v2av[s]);
-            R b1l, b1r, b2l, b2r;
-            if constexpr (MA1) {
-                S::run(ta, c, b1l, b1r);
-                S::run(cur.o, c, b2l, b2r);
-            } else {
-                S::run(cur.o, c, b1l, b1r);
-                S::run(ta, c, b2l, b2r);
-            }
-            const R b1u = pick(sig2, b1l, b1r);
-            const R b2u = pick(sig1, b2l, b2r);
-            R dum = -v1av[s] * b2u + v2av[s] * b1u;
-            // the four cells around the edge (offsets u and w along its
-            // transverse axes, w the march axis): (u-1,w-1) and (u,w-1) are
-            // the previous edge's (u-1,w) and (u,w)
-            const R f_0 = cur.f0, f_u = cur.fu;
-            R eta;
-            if (K == 1)
-                eta = R(.25) * (f_uw + f_w + f_0 + f_u);
-            else if (K == 2)
-                eta = R(.25) * (f_uw + f_u + f_0 + f_w);
-            else
-                eta = R(.25) * (f_uw + f_w + f_0 + f_u);
-            f_uw = f_u;
-            f_w = f_0;
-            dum = dum + eta * (b1l + b2r - b1r - b2l);
-            // ef = |C_a||C_b|/det A of an affine metric (E . a_k per unit
-            // computational length), exactly 1 on the reference's grid; a
-            // general metric gives E . dl per edge (efa)
-            TF ev = TF(dum * (efa ? R(efa[eo]) : ef));
-            step_fence(ev);
-            if (s >= skip) e[eo] = ev;
-            if (s + 1 < T) {
-                if constexpr (!PREB) load_taps(ob1 + omv1, ob2 + omv2, obc + omarch, nxt);
-                cur = nxt;
-            }
-            ob1 += omv1;
-            ob2 += omv2;
-            obc += omarch;
-            eo += ostr;
-        }
-    }
+// the same as part of a launch of several directions (k_stencils): workgroup
+// `part_block` of the direction
+template <typename R, int M, int K, int T, typename TI, typename TF>
+__device__ __forceinline__ void emf_block(Dims d, Coef<R> c, EmfIn<TI> in, R ef, const double* __restrict__ efa,
+                                          TF* __restrict__ e, long nthreads, unsigned part_block) {
+#define EMF_BLOCK() part_block
+#include "mhd_emf_march.inc"
+#undef EMF_BLOCK
 }
 
 }  // namespace mhd

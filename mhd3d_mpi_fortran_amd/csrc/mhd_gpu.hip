@@ -130,6 +130,9 @@ int mhd_create(mhd_ctx** out, const mhd_params* p) {
     // kernels fill the chip for long; small blocks keep one stream
     c->overlap = c->ninterior >= kOverlapCells;
     if (const char* ev = getenv("MHD_EMF_FILL_THREADS")) c->emf_fill = atol(ev);
+    // one launch takes runs of 2 edges, as every EMF of such a block does
+    // unless the fill threshold is lowered
+    c->merged = c->ninterior < kOverlapCells && c->emf_fill >= kEmfFillThreads;
     long nmax = c->ncell;
     nmax = c->nbi > nmax ? c->nbi : nmax;
     nmax = c->nbj > nmax ? c->nbj : nmax;
@@ -831,8 +834,9 @@ static void do_ct_t(mhd_ctx* c, double* const* out) {
 // before the stage ends.  The EMF kernels wait on latency (few waves per
 // SIMD) and CT on HBM, the flux on VALU issue: together they fill the CUs
 // better than one after the other.
-template <int NST, int ST, typename E, typename F>
-static void stage_overlapped(mhd_ctx* c, E emf, F flux, double* const* out) {
+// both: the two in one launch, which blocks below kOverlapCells take (k_stencils)
+template <int NST, int ST, typename E, typename F, typename B>
+static void stage_overlapped(mhd_ctx* c, E emf, F flux, B both, double* const* out) {
     auto cells = [&] {
         if (mixed(c)) do_cells_t<float, NST, ST>(c, out);
         else do_cells_t<double, NST, ST>(c, out);
@@ -846,8 +850,12 @@ static void stage_overlapped(mhd_ctx* c, E emf, F flux, double* const* out) {
     const bool ok = c->overlap && hipEventRecord(c->ev_fork, c->s) == hipSuccess &&
                     hipStreamWaitEvent(c->s2, c->ev_fork, 0) == hipSuccess;
     if (!ok) {   // serial
-        emf();
-        flux();
+        if (c->merged && !c->p.surrogate) {
+            both();
+        } else {
+            emf();
+            flux();
+        }
         if (after_ct) ct();
         cells();
         if (!after_ct) ct();
@@ -934,9 +942,10 @@ static void do_stage(mhd_ctx* c, Src<double> s64, double* const* out) {
         stage_overlapped<NST, ST>(c, [&] { launch_emf_fp32(c, sh_src(c)); }, [&] {
             if (c->p.surrogate) launch_flux_surrogate(c, sh_src(c));
             else launch_flux_fp32(c, sh_src(c));
-        }, out);
+        }, [&] { launch_stage_fp32(c, sh_src(c), kStageFlux | kStageEmf); }, out);
     } else {
-        stage_overlapped<NST, ST>(c, [&] { launch_emf_fp64(c, s64); }, [&] { launch_flux_fp64(c, s64); }, out);
+        stage_overlapped<NST, ST>(c, [&] { launch_emf_fp64(c, s64); }, [&] { launch_flux_fp64(c, s64); },
+                                  [&] { launch_stage_fp64(c, s64, kStageFlux | kStageEmf); }, out);
     }
 }
 

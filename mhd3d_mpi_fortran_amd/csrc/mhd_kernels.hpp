@@ -53,12 +53,15 @@ __device__ __forceinline__ long gtid() { return (long)blockIdx.x * blockDim.x + 
 // points passes 16 / G, so a run always spans 4096 points.
 constexpr unsigned kXcd = 8, kXcdRun = 16;
 template <unsigned RUN = kXcdRun>
-__device__ __forceinline__ unsigned xcd_block() {
-    const unsigned b = blockIdx.x, n = gridDim.x;
+__device__ __forceinline__ unsigned xcd_map(unsigned b, unsigned n) {
     const unsigned base = b / (kXcd * RUN) * (kXcd * RUN), r = b - base;
     const unsigned m = n - base < kXcd * RUN ? n - base : kXcd * RUN;
     const unsigned n8 = m / kXcd, rem = m % kXcd, x = r % kXcd, q = r / kXcd;
     return base + x * n8 + (x < rem ? x : rem) + q;
+}
+template <unsigned RUN = kXcdRun>
+__device__ __forceinline__ unsigned xcd_block() {
+    return xcd_map<RUN>(blockIdx.x, gridDim.x);
 }
 __device__ __forceinline__ long gtid_xcd() { return (long)xcd_block() * blockDim.x + threadIdx.x; }
 
@@ -319,14 +322,19 @@ __host__ __device__ __forceinline__ unsigned face_runs(int ii, int jj, int kk, i
     const unsigned ntn = (nn + kTileN - 1) / kTileN;
     return (unsigned)((ii + kTileX - 1) / kTileX) * ((ntn + run - 1) / run) * no;
 }
+template <typename R, int M, typename TI, int RUN>
+struct FluxRing {  // the rows in LDS (binary64 sweeps use none)
+    static constexpr int NR = kTileN + Stencil<R, M>::n - 1;
+    static constexpr int RING = RUN == 1 ? NR : kFluxRing;
+    static_assert(NR <= kFluxRing, "the ring holds one tile's rows");
+    using Win = TI[sizeof(TI) == 4 ? 8 : 1][sizeof(TI) == 4 ? RING : 1][kTileX];
+};
 template <typename R, int M, int D, typename TI, int RUN>
 __device__ __forceinline__ void ring_recon(const Dims& d, const Prim<TI>& q, const Coef<R>& c, unsigned tx,
-                                           unsigned tn, unsigned o, int ii, unsigned no, bool first, R* l, R* r) {
+                                           unsigned tn, unsigned o, int ii, unsigned no, bool first,
+                                           typename FluxRing<R, M, TI, RUN>::Win& win, R* l, R* r) {
     using S = Stencil<R, M>;
-    constexpr int NR = kTileN + S::n - 1;
-    constexpr int RING = RUN == 1 ? NR : kFluxRing;
-    static_assert(NR <= kFluxRing, "the ring holds one tile's rows");
-    __shared__ TI win[8][RING][kTileX];
+    constexpr int NR = FluxRing<R, M, TI, RUN>::NR;
     // LDS slot of the tile's row rho
     auto slot = [&](int rho) { return RUN == 1 ? rho : ((int)(tn * kTileN) + rho) & (kFluxRing - 1); };
     const TI* f[8] = {q.rho, q.vx, q.vy, q.vz, q.p, q.bx, q.by, q.bz};
@@ -356,9 +364,11 @@ __device__ __forceinline__ void ring_recon(const Dims& d, const Prim<TI>& q, con
 // MET = 0: the reference's axis-aligned flux; 1: along the affine metric's
 // normals; 2: along the general metric's per-face normals
 // RUN: face tiles per workgroup of the fp32 strided sweeps
-template <typename R, int M, int D, typename TI, typename TF, int MET, int RUN = 1>
-__global__ void __launch_bounds__(kBlock) k_flux(Dims d, Coef<R> c, Prim<TI> q, Normals<R> nm, GMet gm,
-                                                 TF* __restrict__ F, long nface) {
+// lb: the workgroup's place in the direction's own order; win: the kernel's LDS rows
+template <typename R, int M, int D, typename TI, typename TF, int MET, int RUN>
+__device__ __forceinline__ void flux_block(const Dims& d, const Coef<R>& c, const Prim<TI>& q, const Normals<R>& nm,
+                                           const GMet& gm, TF* __restrict__ F, long nface, unsigned lb,
+                                           typename FluxRing<R, M, TI, RUN>::Win& win) {
     const int ii = d.nx0 + (D == 1), jj = d.ny0 + (D == 2), kk = d.nz0 + (D == 3);
     const ptrdiff_t st = D == 1 ? 1 : (D == 2 ? (ptrdiff_t)d.nx : (ptrdiff_t)d.nx * d.ny);
     int i, j, k;
@@ -367,7 +377,7 @@ __global__ void __launch_bounds__(kBlock) k_flux(Dims d, Coef<R> c, Prim<TI> q, 
     if constexpr (D == 1) {
         // flat; unit stride: the taps of one array are contiguous and load
         // as wide vectors from one address
-        t = gtid_xcd();
+        t = (long)lb * kBlock + threadIdx.x;
         if (t >= nface) return;
         unflat(t, ii, jj, i, j, k);
         const ptrdiff_t base = ix(d.nx, d.ny, d.ng + i, d.ng + j, d.ng + k);
@@ -385,13 +395,12 @@ __global__ void __launch_bounds__(kBlock) k_flux(Dims d, Coef<R> c, Prim<TI> q, 
         const unsigned nn = D == 2 ? jj : kk, no = D == 2 ? kk : jj;
         const unsigned ntx = (ii + kTileX - 1) / kTileX, ntn = (nn + kTileN - 1) / kTileN;
         const unsigned ntc = (ntn + RUN - 1) / RUN;
-        const unsigned lb = xcd_block<kXcdRun / RUN>();
         const unsigned tx = lb % ntx, tnc = lb / ntx % ntc, o = lb / ntx / ntc;
         const unsigned x = tx * kTileX + (threadIdx.x & (kTileX - 1));
 #pragma unroll 1
         for (int g = 0; g < RUN; ++g) {
             const unsigned tn = tnc * RUN + g, sw = tn * kTileN + threadIdx.x / kTileX;
-            ring_recon<R, M, D, TI, RUN>(d, q, c, tx, tn, o, ii, no, g == 0, l, r);
+            ring_recon<R, M, D, TI, RUN>(d, q, c, tx, tn, o, ii, no, g == 0, win, l, r);
             if (x < (unsigned)ii && sw < nn) {
                 i = (int)x + 1;
                 j = (int)(D == 2 ? sw : o) + 1;
@@ -411,7 +420,7 @@ __global__ void __launch_bounds__(kBlock) k_flux(Dims d, Coef<R> c, Prim<TI> q, 
         return;
     } else {
         // binary64 (VALU-bound): taps from the tile's rows in L1
-        if (!tile_face<D>(xcd_block(), ii, jj, kk, i, j, k)) return;
+        if (!tile_face<D>(lb, ii, jj, kk, i, j, k)) return;
         t = ix(ii, jj, i, j, k);
         const Taps<R, M, TI> tp(ix(d.nx, d.ny, d.ng + i, d.ng + j, d.ng + k), st);
         recon_taps<R, M>(q.rho, tp, c, l[0], r[0]);
@@ -432,6 +441,14 @@ __global__ void __launch_bounds__(kBlock) k_flux(Dims d, Coef<R> c, Prim<TI> q, 
     } else {
         face_flux<R, D, TF>(c, l, r, F, t, nface);
     }
+}
+
+template <typename R, int M, int D, typename TI, typename TF, int MET, int RUN = 1>
+__global__ void __launch_bounds__(kBlock) k_flux(Dims d, Coef<R> c, Prim<TI> q, Normals<R> nm, GMet gm,
+                                                 TF* __restrict__ F, long nface) {
+    __shared__ typename FluxRing<R, M, TI, RUN>::Win win;
+    const unsigned lb = D != 1 && sizeof(TI) == 4 ? xcd_block<kXcdRun / RUN>() : xcd_block();
+    flux_block<R, M, D, TI, TF, MET, RUN>(d, c, q, nm, gm, F, nface, lb, win);
 }
 
 // ------------------------------------------------------------------------

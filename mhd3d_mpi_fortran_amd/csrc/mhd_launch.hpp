@@ -67,6 +67,7 @@ struct mhd_ctx {
     // targets (null = s)
     hipStream_t s2 = nullptr, cur = nullptr;
     hipEvent_t ev_fork = nullptr, ev_emf = nullptr, ev_join = nullptr;
+    bool merged = false;   // one launch for a stage's stencils (blocks below kOverlapCells)
     bool overlap = true;   // false: one stream, kernels in the reference's order
     bool fused = false;    // mixed Adams-Bashforth PDM steps: fused face flux + update (mhd_set_fusion)
     char* arena = nullptr;
@@ -205,6 +206,10 @@ void launch_emf_fp64(mhd_ctx* c, mhd::Src<double> s);
 void launch_recon(mhd_ctx* c, int dir, const double* f, int fn1, int fn2, int lnx, int lny, int lnz, double* fl,
                   double* fr);
 void launch_flux_fp32(mhd_ctx* c, mhd::Src<float> s);
+// the face fluxes and/or the edge EMFs in one launch (k_stencils)
+enum { kStageFlux = 1, kStageEmf = 2 };
+void launch_stage_fp64(mhd_ctx* c, mhd::Src<double> s, int what);
+void launch_stage_fp32(mhd_ctx* c, mhd::Src<float> s, int what);
 void launch_emf_fp32(mhd_ctx* c, mhd::Src<float> s);
 void launch_flux_surrogate(mhd_ctx* c, mhd::Src<float> s);
 void launch_vface_fp64(mhd_ctx* c, long n, const double* lam, const double* v, double* v0p, double* v0n, double* v1p,

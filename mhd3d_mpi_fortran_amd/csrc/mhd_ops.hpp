@@ -9,6 +9,72 @@
 
 namespace mhd {
 
+// edges handled per thread along the march axis: long runs share the
+// sliding stencil windows; a launch whose long-run grid has fewer threads
+// than c->emf_fill takes runs of 2 instead, trading window reuse for latency
+// hiding.  PDM's ei march (both corner axes strided, its loads the slowest)
+// takes runs of 16: at 256^3 0.20 vs 0.22 ms (fp32) and 0.48 vs 0.51 ms
+// (binary64), and runs of 32 are slower again (0.23 ms fp32, 0.83 ms
+// binary64); for ej and ek runs of 16 measured slower (0.19 vs 0.17 ms
+// fp32), and so did runs of 4 (0.17 vs 0.16 ms) and register caps that
+// buy a fifth or sixth wavefront per SIMD with spills (EMF class 0.61 and
+// 0.72 vs 0.53 ms).
+template <int M, int K>
+struct EmfSteps {
+    static constexpr int T = (M == TVD || (M == PDM && K == 1)) ? 16 : 8;
+    static constexpr int T_SHORT = 2;
+};
+
+// Small and ordinary blocks: the face fluxes and edge EMFs of a stage in one
+// launch.  They are independent, and on such blocks each kernel alone neither
+// fills the chip (64^3: 500-1100 workgroups of one direction on 256 CUs) nor
+// lives long enough to hide its own start and tail, so one after the other they
+// take several times what their arithmetic needs.  The grid is the six
+// kernels' workgroups end to end, the EMF's (the longest) first; every
+// workgroup belongs to one of them.  Its registers are the largest of the six,
+// which large blocks would pay for in the flux: they keep the separate
+// kernels, EMF and flux on two streams.  A stage of 64^3 (PDM, binary64) took
+// 114 us with the six kernels and takes 84 us, 16^3 51 and 12 us.
+template <typename R, typename TF>
+struct StencilOut {
+    TF* flux[3];
+    TF* emf[3];
+    long nface[3];
+    R ef[3];
+    const double* efa[3];
+    long nthreads[3];      // EMF threads per direction
+    unsigned end[6];       // last workgroup + 1 of the EMF's and the flux's directions
+};
+template <typename R, int M, typename TI, typename TF, int MET, bool EMF>
+__global__ void __launch_bounds__(kBlock) k_stencils(Dims d, Coef<R> c, Prim<TI> q, Normals<R> nm, GMet gm,
+                                                    EmfIn<TI> e1, EmfIn<TI> e2, EmfIn<TI> e3,
+                                                    StencilOut<R, TF> o) {
+    __shared__ typename FluxRing<R, M, TI, 1>::Win win;
+    const unsigned b = blockIdx.x;
+    auto place = [&](int p) {  // place within part p, in its XCD-aware order
+        const unsigned lo = p ? o.end[p - 1] : 0;
+        return xcd_map(b - lo, o.end[p] - lo);
+    };
+    constexpr int T = EmfSteps<M, 1>::T_SHORT;
+    if constexpr (EMF) {
+        if (b < o.end[0]) {
+            emf_block<R, M, 1, T, TI, TF>(d, c, e1, o.ef[0], o.efa[0], o.emf[0], o.nthreads[0], place(0));
+            return;
+        }
+        if (b < o.end[1]) {
+            emf_block<R, M, 2, T, TI, TF>(d, c, e2, o.ef[1], o.efa[1], o.emf[1], o.nthreads[1], place(1));
+            return;
+        }
+        if (b < o.end[2]) {
+            emf_block<R, M, 3, T, TI, TF>(d, c, e3, o.ef[2], o.efa[2], o.emf[2], o.nthreads[2], place(2));
+            return;
+        }
+    }
+    if (b < o.end[3]) flux_block<R, M, 2, TI, TF, MET, 1>(d, c, q, nm, gm, o.flux[1], o.nface[1], place(3), win);
+    else if (b < o.end[4]) flux_block<R, M, 3, TI, TF, MET, 1>(d, c, q, nm, gm, o.flux[2], o.nface[2], place(4), win);
+    else flux_block<R, M, 1, TI, TF, MET, 1>(d, c, q, nm, gm, o.flux[0], o.nface[0], place(5), win);
+}
+
 template <typename R, typename TI, typename TF, int M, int MET>
 void flux_launch_mm(mhd_ctx* c, Src<TI> s) {
     const Coef<R> co = make_coef<R>(c);
@@ -52,22 +118,6 @@ void flux_launch(mhd_ctx* c, Src<TI> s) {
     default: flux_launch_m<R, TI, TF, MPWENO5>(c, s); break;
     }
 }
-
-// edges handled per thread along the march axis: long runs share the
-// sliding stencil windows; a launch whose long-run grid has fewer threads
-// than c->emf_fill takes runs of 2 instead, trading window reuse for latency
-// hiding.  PDM's ei march (both corner axes strided, its loads the slowest)
-// takes runs of 16: at 256^3 0.20 vs 0.22 ms (fp32) and 0.48 vs 0.51 ms
-// (binary64), and runs of 32 are slower again (0.23 ms fp32, 0.83 ms
-// binary64); for ej and ek runs of 16 measured slower (0.19 vs 0.17 ms
-// fp32), and so did runs of 4 (0.17 vs 0.16 ms) and register caps that
-// buy a fifth or sixth wavefront per SIMD with spills (EMF class 0.61 and
-// 0.72 vs 0.53 ms).
-template <int M, int K>
-struct EmfSteps {
-    static constexpr int T = (M == TVD || (M == PDM && K == 1)) ? 16 : 8;
-    static constexpr int T_SHORT = 2;
-};
 
 template <typename R, int M, int K, int T, typename TI, typename TF>
 void emf_launch_kt(mhd_ctx* c, EmfIn<TI> in) {
@@ -152,6 +202,65 @@ void emf_launch(mhd_ctx* c, Src<TI> s) {
     case TVD: emf_launch_m<R, TI, TF, TVD>(c, s); break;
     case WENO5: emf_launch_m<R, TI, TF, WENO5>(c, s); break;
     default: emf_launch_m<R, TI, TF, MPWENO5>(c, s); break;
+    }
+}
+
+// a stage's stencils in one launch (what: kStageFlux | kStageEmf)
+template <typename R, typename TI, typename TF, int M, int MET>
+void stage_launch_mm(mhd_ctx* c, Src<TI> s, int what) {
+    const Dims& d = c->d;
+    constexpr bool march = M == PDM || M == TVD;
+    constexpr int T = EmfSteps<M, 1>::T_SHORT;
+    StencilOut<R, TF> o{};
+    unsigned nb[6] = {0, 0, 0, 0, 0, 0};
+    for (int a = 0; a < 3; ++a) {
+        o.flux[a] = (TF*)c->flux[a];
+        o.emf[a] = (TF*)c->emf[a];
+        o.nface[a] = c->nf[a];
+        o.ef[a] = R(c->met.ef[a]);
+        o.efa[a] = c->met.mode == 2 ? c->gm.ef[a] : nullptr;
+    }
+    if ((what & kStageEmf) && march) {
+        for (int a = 0; a < 3; ++a) {
+            const long ii = d.nx0 + (a != 0), no = a == 2 ? d.nz0 : (a == 0 ? d.ny0 + 1 : d.ny0);
+            const long nm = a == 2 ? d.ny0 + 1 : d.nz0 + 1;
+            o.nthreads[a] = ii * no * ((nm + T - 1) / T);
+            nb[a] = a == 0 ? emf_tiles<T>(d.nx0, d.ny0, d.nz0) : blocks(o.nthreads[a]).x;
+        }
+    }
+    if (what & kStageFlux) {
+        nb[3] = face_tiles<2>(d.nx0, d.ny0 + 1, d.nz0);
+        nb[4] = face_tiles<3>(d.nx0, d.ny0, d.nz0 + 1);
+        nb[5] = blocks(c->nf[0]).x;
+    }
+    unsigned n = 0;
+    for (int a = 0; a < 6; ++a) o.end[a] = n += nb[a];
+    const Prim<TI> q{s.rho, s.vx, s.vy, s.vz, s.p, s.bx, s.by, s.bz};
+    const TI* u[3] = {s.vx, s.vy, s.vz};
+    if (c->met.on)
+        for (int a = 0; a < 3; ++a) u[a] = s.w[a];
+    launch(c, what & kStageFlux ? MHD_K_FLUX : MHD_K_EMF, dim3(n), dim3(kBlock), k_stencils<R, M, TI, TF, MET, march>, d,
+           make_coef<R>(c), q, make_normals<R>(c), c->gm, EmfIn<TI>{u[1], u[2], s.bj, s.bk, s.vf},
+           EmfIn<TI>{u[2], u[0], s.bk, s.bi, s.vf}, EmfIn<TI>{u[0], u[1], s.bi, s.bj, s.vf}, o);
+    if constexpr (!march) {
+        if (what & kStageEmf) emf_launch_m<R, TI, TF, M>(c, s);
+    }
+}
+
+template <typename R, typename TI, typename TF, int M>
+void stage_launch_m(mhd_ctx* c, Src<TI> s, int what) {
+    if (c->met.mode == 2) stage_launch_mm<R, TI, TF, M, 2>(c, s, what);
+    else if (c->met.on) stage_launch_mm<R, TI, TF, M, 1>(c, s, what);
+    else stage_launch_mm<R, TI, TF, M, 0>(c, s, what);
+}
+
+template <typename R, typename TI, typename TF>
+void stage_launch(mhd_ctx* c, Src<TI> s, int what) {
+    switch (c->p.reconop) {
+    case PDM: stage_launch_m<R, TI, TF, PDM>(c, s, what); break;
+    case TVD: stage_launch_m<R, TI, TF, TVD>(c, s, what); break;
+    case WENO5: stage_launch_m<R, TI, TF, WENO5>(c, s, what); break;
+    default: stage_launch_m<R, TI, TF, MPWENO5>(c, s, what); break;
     }
 }
 

@@ -5,9 +5,18 @@
 
 using namespace mhd;
 
-void launch_flux_fp32(mhd_ctx* c, Src<float> s) { flux_launch<float, float, float>(c, s); }
+void launch_stage_fp32(mhd_ctx* c, Src<float> s, int what) { stage_launch<float, float, float>(c, s, what); }
 
-void launch_emf_fp32(mhd_ctx* c, Src<float> s) { emf_launch<float, float, float>(c, s); }
+// (a block's kernels are the same however its stencils are asked for)
+void launch_flux_fp32(mhd_ctx* c, Src<float> s) {
+    if (c->merged) launch_stage_fp32(c, s, kStageFlux);
+    else flux_launch<float, float, float>(c, s);
+}
+
+void launch_emf_fp32(mhd_ctx* c, Src<float> s) {
+    if (c->merged) launch_stage_fp32(c, s, kStageEmf);
+    else emf_launch<float, float, float>(c, s);
+}
 
 void launch_vface_fp32(mhd_ctx* c, long n, const double* lam, const double* v, double* v0p, double* v0n, double* v1p,
                      double* v1n) {

@@ -5,9 +5,18 @@
 
 using namespace mhd;
 
-void launch_flux_fp64(mhd_ctx* c, Src<double> s) { flux_launch<double, double, double>(c, s); }
+void launch_stage_fp64(mhd_ctx* c, Src<double> s, int what) { stage_launch<double, double, double>(c, s, what); }
 
-void launch_emf_fp64(mhd_ctx* c, Src<double> s) { emf_launch<double, double, double>(c, s); }
+// (a block's kernels are the same however its stencils are asked for)
+void launch_flux_fp64(mhd_ctx* c, Src<double> s) {
+    if (c->merged) launch_stage_fp64(c, s, kStageFlux);
+    else flux_launch<double, double, double>(c, s);
+}
+
+void launch_emf_fp64(mhd_ctx* c, Src<double> s) {
+    if (c->merged) launch_stage_fp64(c, s, kStageEmf);
+    else emf_launch<double, double, double>(c, s);
+}
 
 void launch_recon(mhd_ctx* c, int dir, const double* f, int fn1, int fn2, int lnx, int lny, int lnz, double* fl,
                   double* fr) {
