@@ -117,14 +117,12 @@ __device__ __forceinline__ float rough5(const float* x) {
 
 struct State {
     float* p = nullptr;        // fp32 master parameters
-    float* g = nullptr;        // gradient accumulator
     float* m = nullptr;        // Adam moments
     float* v = nullptr;
     float* samples = nullptr;  // [cap][NS]
     long cap = 0;
     long* count = nullptr;     // device counter of collected samples
-    float* scratch = nullptr;  // per-sample activations/deltas of one minibatch
-    long scratch_n = 0;
+    float* scratch = nullptr;  // per-chunk gradient sums and squared errors of one minibatch
     float* loss = nullptr;     // device loss accumulator
     unsigned short* wbf = nullptr;  // bf16 MFMA A operands per lane (k_pack_bf16)
     float* bias = nullptr;     // biases in D-register order per half-wave (fp32)
@@ -246,127 +244,165 @@ __global__ void __launch_bounds__(1024) k_collect_scan(const long* __restrict__ 
 
 // ---------------------------------------------------------------------------
 // training
-// scratch per sample b: x(40) a1(32) a2(32) dz1(32) dz2(32) dy(16)
 // ---------------------------------------------------------------------------
-constexpr int SC = NI + 4 * NH + NO;  // 184
+// Forward, backward and gradient of one minibatch: kGradChunks workgroups, each
+// a run of consecutive samples, kTrainTile of them at a time.  Sample b of
+// the batch is sample (first + b*mult) mod n of the set (a permutation when
+// gcd(mult, n) = 1).
+//
+// 32 lanes work on a sample, one per unit of a layer: a lane adds its unit's
+// products in the order of the inputs, reading its row of weights and the
+// layer's inputs (the same word for all 32) from LDS.  Rows are padded to an odd
+// length, so that rows (forward) and columns (backward) are both read without
+// bank conflicts.  The deltas and activations of a tile stay in LDS, and each
+// thread then adds them up for 6 of the 2896 parameters, in sample order.  A
+// chunk's partial sums go to a slot of its own and k_grad_sum / k_grad_adam add
+// the slots in chunk order, so the gradient -- and the training -- does not
+// depend on the order in which the workgroups finish.
+//
+// One thread a sample (4 workgroups for a batch of 1024, the layers in
+// per-thread arrays that spilled 8.6 KB to scratch memory, and a second pass over
+// the activations in HBM) took 167 + 7 us a minibatch of 1024, and 9.7 us for the
+// sums and Adam; this takes 10.8 us and k_grad_adam 4.2 us.  Bound: the latency
+// of the layers' serial sums and of LDS; the arithmetic is 18 Mflop.
+constexpr int kGradChunks = 64;
+constexpr int kTrainTile = 16, kTrainThreads = 32 * kTrainTile;
+// a sample's words in LDS: x(40) a1(32) a2(32) dz1(32) dz2(32) dy(16)
+constexpr int T_A1 = NI, T_A2 = T_A1 + NH, T_D1 = T_A2 + NH, T_D2 = T_D1 + NH, T_DY = T_D2 + NH, T_N = T_DY + NO;
 
-// forward + backward of one minibatch; sample b of the batch is sample
-// (first + b*mult) mod n of the set (a permutation when gcd(mult, n) = 1)
-__global__ void __launch_bounds__(kBlock) k_train_fb(const float* __restrict__ P, const float* __restrict__ set,
-                                                    long n, long first, long mult, int batch, float inv_norm,
-                                                    float* __restrict__ scratch, float* __restrict__ loss) {
-    __shared__ float w[NPARAM];
-    for (int a = threadIdx.x; a < NPARAM; a += blockDim.x) w[a] = P[a];
-    __syncthreads();
-    const int b = blockIdx.x * blockDim.x + threadIdx.x;
+__global__ void __launch_bounds__(kTrainThreads) k_train(const float* __restrict__ P, const float* __restrict__ set,
+                                                         long n, long first, long mult, int batch, float inv_norm,
+                                                         float* __restrict__ gpart, float* __restrict__ lpart) {
+    constexpr int R1 = NI + 1, R2 = NH + 1;  // padded rows
+    __shared__ float w1[NH * R1], w2[NH * R2], w3[NO * R2], bias[2 * NH + NO], sc[kTrainTile][T_N];
+    __shared__ float red[kTrainThreads / 64];
+    const int tid = threadIdx.x, s = tid >> 5, j = tid & 31;
+    for (int a = tid; a < NH * NI; a += kTrainThreads) w1[a / NI * R1 + a % NI] = P[OFF_W1 + a];
+    for (int a = tid; a < NH * NH; a += kTrainThreads) w2[a / NH * R2 + a % NH] = P[OFF_W2 + a];
+    for (int a = tid; a < NO * NH; a += kTrainThreads) w3[a / NH * R2 + a % NH] = P[OFF_W3 + a];
+    if (tid < NH) {
+        bias[tid] = P[OFF_B1 + tid];
+        bias[NH + tid] = P[OFF_B2 + tid];
+        if (tid < NO) bias[2 * NH + tid] = P[OFF_B3 + tid];
+    }
+    // this thread's parameters: the delta and the activation their gradient
+    // multiplies (activation -1: a bias)
+    constexpr int NP = (NPARAM + kTrainThreads - 1) / kTrainThreads;
+    int din[NP], ain[NP];
+    float g[NP];
+#pragma unroll
+    for (int q = 0; q < NP; ++q) {
+        const int p = tid + q * kTrainThreads;
+        g[q] = 0.f;
+        ain[q] = -1;
+        if (p < OFF_B1) { din[q] = T_D1 + p / NI; ain[q] = p % NI; }
+        else if (p < OFF_W2) din[q] = T_D1 + (p - OFF_B1);
+        else if (p < OFF_B2) { din[q] = T_D2 + (p - OFF_W2) / NH; ain[q] = T_A1 + (p - OFF_W2) % NH; }
+        else if (p < OFF_W3) din[q] = T_D2 + (p - OFF_B2);
+        else if (p < OFF_B3) { din[q] = T_DY + (p - OFF_W3) / NH; ain[q] = T_A2 + (p - OFF_W3) % NH; }
+        else din[q] = p < NPARAM ? T_DY + (p - OFF_B3) : 0;
+    }
+    const int per = (batch + kGradChunks - 1) / kGradChunks;
+    const int b0 = min((int)blockIdx.x * per, batch), b1 = min(b0 + per, batch);
     float l2 = 0.f;
-    if (b < batch) {
-        const long idx = (long)(((unsigned long long)first + (unsigned long long)b * (unsigned long long)mult) % (unsigned long long)n);
-        const float* s = set + idx * NS;
-        float* sc = scratch + (long)b * SC;
-        float x[NI], z1[NH], a1[NH], z2[NH], a2[NH], y[NO];
-        for (int a = 0; a < NI; ++a) {
-            x[a] = s[a];
-            sc[a] = x[a];
+    for (int t0 = b0; t0 < b1; t0 += kTrainTile) {
+        const int b = t0 + s;
+        const bool live = b < b1;
+        float target = 0.f;
+        float* x = sc[s];
+        {
+            const long idx = (long)(((unsigned long long)first + (unsigned long long)(live ? b : b0) *
+                                                                     (unsigned long long)mult) %
+                                    (unsigned long long)n);
+            const float* from = set + idx * NS;
+            x[j] = from[j];
+            if (j < NI - 32) x[32 + j] = from[32 + j];
+            if (j < NO) target = from[NI + j];
         }
-        for (int j = 0; j < NH; ++j) {
-            float acc = w[OFF_B1 + j];
-            for (int a = 0; a < NI; ++a) acc += w[OFF_W1 + j * NI + a] * x[a];
-            z1[j] = acc;
-            a1[j] = act(acc);
-            sc[NI + j] = a1[j];
+        __syncthreads();
+        float z1 = bias[j];
+        for (int a = 0; a < NI; ++a) z1 += w1[j * R1 + a] * x[a];
+        x[T_A1 + j] = act(z1);
+        __syncthreads();
+        float z2 = bias[NH + j];
+        for (int a = 0; a < NH; ++a) z2 += w2[j * R2 + a] * x[T_A1 + a];
+        x[T_A2 + j] = act(z2);
+        __syncthreads();
+        if (j < NO) {
+            float acc = bias[2 * NH + j];
+            for (int a = 0; a < NH; ++a) acc += w3[j * R2 + a] * x[T_A2 + a];
+            const float gt = rough5(x + 5 * (j & 7));
+            const float e = lin4(x + 5 * (j & 7)) + gt * acc - target;
+            if (live) l2 += e * e;
+            x[T_DY + j] = 2.f * e * gt * inv_norm;
         }
-        for (int j = 0; j < NH; ++j) {
-            float acc = w[OFF_B2 + j];
-            for (int a = 0; a < NH; ++a) acc += w[OFF_W2 + j * NH + a] * a1[a];
-            z2[j] = acc;
-            a2[j] = act(acc);
-            sc[NI + NH + j] = a2[j];
-        }
-        float dy[NO];
-        for (int o = 0; o < NO; ++o) {
-            float acc = w[OFF_B3 + o];
-            for (int a = 0; a < NH; ++a) acc += w[OFF_W3 + o * NH + a] * a2[a];
-            const float gt = rough5(x + 5 * (o & 7));
-            y[o] = lin4(x + 5 * (o & 7)) + gt * acc;
-            const float e = y[o] - s[NI + o];
-            l2 += e * e;
-            dy[o] = 2.f * e * gt * inv_norm;
-            sc[NI + 4 * NH + o] = dy[o];
-        }
-        float dz2[NH];
-        for (int a = 0; a < NH; ++a) {
+        __syncthreads();
+        {
             float acc = 0.f;
-            for (int o = 0; o < NO; ++o) acc += w[OFF_W3 + o * NH + a] * dy[o];
-            dz2[a] = acc * act_grad(z2[a]);
-            sc[NI + 3 * NH + a] = dz2[a];
+            for (int o = 0; o < NO; ++o) acc += w3[o * R2 + j] * x[T_DY + o];
+            x[T_D2 + j] = acc * act_grad(z2);
         }
-        for (int a = 0; a < NH; ++a) {
+        __syncthreads();
+        {
             float acc = 0.f;
-            for (int j = 0; j < NH; ++j) acc += w[OFF_W2 + j * NH + a] * dz2[j];
-            sc[NI + 2 * NH + a] = acc * act_grad(z1[a]);
+            for (int o = 0; o < NH; ++o) acc += w2[o * R2 + j] * x[T_D2 + o];
+            x[T_D1 + j] = acc * act_grad(z1);
         }
+        __syncthreads();
+        const int m = min(kTrainTile, b1 - t0);
+#pragma unroll
+        for (int q = 0; q < NP; ++q)
+            for (int u = 0; u < m; ++u) g[q] += sc[u][din[q]] * (ain[q] >= 0 ? sc[u][ain[q]] : 1.f);
+        __syncthreads();
     }
-    // block sum of the squared error
-    __shared__ float red[kBlock / 64];
+#pragma unroll
+    for (int q = 0; q < NP; ++q) {
+        const int p = tid + q * kTrainThreads;
+        if (p < NPARAM) gpart[(long)blockIdx.x * NPARAM + p] = g[q];
+    }
     for (int o = 32; o > 0; o >>= 1) l2 += __shfl_xor(l2, o, 64);
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = l2;
+    if ((tid & 63) == 0) red[tid >> 6] = l2;
     __syncthreads();
-    if (threadIdx.x == 0) {
-        float s = 0.f;
-        for (int q = 0; q < (int)(blockDim.x >> 6); ++q) s += red[q];
-        atomicAdd(loss, s);
+    if (tid == 0) {
+        float t = 0.f;
+        for (int q = 0; q < kTrainThreads / 64; ++q) t += red[q];
+        lpart[blockIdx.x] = t;
     }
 }
 
-// dParam = sum over the batch of delta_out * activation_in; each workgroup
-// covers 64 parameters x 4 batch chunks, grid.y splits the batch further.
-// Each chunk's partial sum goes to a slot of its own and k_grad_sum adds the
-// kGradChunks slots in chunk order, so the gradient -- and the training --
-// does not depend on the order in which the chunks finish.
-constexpr int kGradChunks = 64;  // = grid.y (16) x 4 wavefronts
-__global__ void __launch_bounds__(kBlock) k_train_grad(const float* __restrict__ scratch, int batch,
-                                                      float* __restrict__ gpart) {
-    const int pidx = blockIdx.x * 64 + (threadIdx.x & 63);
-    const int nch = gridDim.y * 4;
-    const int ch = blockIdx.y * 4 + (threadIdx.x >> 6);
-    if (pidx >= NPARAM) return;
-    int din, ain;  // scratch offsets of delta and input activation (-1: bias)
-    if (pidx < OFF_B1) { din = NI + 2 * NH + pidx / NI; ain = pidx % NI; }
-    else if (pidx < OFF_W2) { din = NI + 2 * NH + (pidx - OFF_B1); ain = -1; }
-    else if (pidx < OFF_B2) { din = NI + 3 * NH + (pidx - OFF_W2) / NH; ain = NI + (pidx - OFF_W2) % NH; }
-    else if (pidx < OFF_W3) { din = NI + 3 * NH + (pidx - OFF_B2); ain = -1; }
-    else if (pidx < OFF_B3) { din = NI + 4 * NH + (pidx - OFF_W3) / NH; ain = NI + NH + (pidx - OFF_W3) % NH; }
-    else { din = NI + 4 * NH + (pidx - OFF_B3); ain = -1; }
-    const int per = (batch + nch - 1) / nch;
-    const int b0 = ch * per, b1 = b0 + per < batch ? b0 + per : batch;
-    float acc = 0.f;
-    for (int b = b0; b < b1; ++b) {
-        const float* sc = scratch + (long)b * SC;
-        acc += sc[din] * (ain >= 0 ? sc[ain] : 1.f);
-    }
-    gpart[(long)ch * NPARAM + pidx] = acc;
-}
-
-__global__ void k_grad_sum(const float* __restrict__ gpart, float* __restrict__ g) {
-    const int a = blockIdx.x * blockDim.x + threadIdx.x;
-    if (a >= NPARAM) return;
+// the chunks' partial sums of parameter a, in chunk order; the first thread
+// adds the chunks' squared errors to the loss
+__device__ __forceinline__ float grad_of(const float* __restrict__ gpart, const float* __restrict__ lpart, int a,
+                                         float* __restrict__ loss) {
     float s = 0.f;
+#pragma unroll 16
     for (int ch = 0; ch < kGradChunks; ++ch) s += gpart[(long)ch * NPARAM + a];
-    g[a] = s;
+    if (a == 0) {
+        float t = 0.f;
+        for (int ch = 0; ch < kGradChunks; ++ch) t += lpart[ch];
+        *loss += t;
+    }
+    return s;
 }
 
-__global__ void k_adam(float* __restrict__ P, float* __restrict__ g, float* __restrict__ m, float* __restrict__ v,
-                       float lr, float b1c, float b2c) {
+__global__ void k_grad_sum(const float* __restrict__ gpart, const float* __restrict__ lpart, float* __restrict__ g,
+                           float* __restrict__ loss) {
+    const int a = blockIdx.x * blockDim.x + threadIdx.x;
+    if (a < NPARAM) g[a] = grad_of(gpart, lpart, a, loss);
+}
+
+// the same and Adam's step: one launch a minibatch after k_train
+__global__ void k_grad_adam(const float* __restrict__ gpart, const float* __restrict__ lpart, float* __restrict__ P,
+                            float* __restrict__ m, float* __restrict__ v, float lr, float b1c, float b2c,
+                            float* __restrict__ loss) {
     const int a = blockIdx.x * blockDim.x + threadIdx.x;
     if (a >= NPARAM) return;
-    const float gg = g[a];
+    const float gg = grad_of(gpart, lpart, a, loss);
     const float mm = .9f * m[a] + .1f * gg;
     const float vv = .999f * v[a] + .001f * gg * gg;
     m[a] = mm;
     v[a] = vv;
     P[a] -= lr * (mm / b1c) / (sqrtf(vv / b2c) + 1e-8f);
-    g[a] = 0.f;
 }
 
 __global__ void k_zero_f(float* __restrict__ p, int n) {
@@ -966,7 +1002,7 @@ static SurrogateState* sstate(mhd_ctx* c) {
     if (!c->sur) {
         SurrogateState* s = new SurrogateState();
         const size_t pb = sur::NPARAM * sizeof(float);
-        bool ok = hipMalloc(&s->p, pb) == hipSuccess && hipMalloc(&s->g, pb) == hipSuccess &&
+        bool ok = hipMalloc(&s->p, pb) == hipSuccess &&
                   hipMalloc(&s->m, pb) == hipSuccess && hipMalloc(&s->v, pb) == hipSuccess &&
                   hipMalloc(&s->count, 64) == hipSuccess && hipMalloc(&s->loss, 64) == hipSuccess &&
                   hipMalloc(&s->wbf, sur::WBF_N * sizeof(unsigned short)) == hipSuccess &&
@@ -977,7 +1013,7 @@ static SurrogateState* sstate(mhd_ctx* c) {
             return nullptr;
         }
         c->sur = s;
-        if (hipMemsetAsync(s->g, 0, pb, c->s) != hipSuccess || hipMemsetAsync(s->m, 0, pb, c->s) != hipSuccess ||
+        if (hipMemsetAsync(s->m, 0, pb, c->s) != hipSuccess ||
             hipMemsetAsync(s->v, 0, pb, c->s) != hipSuccess || hipMemsetAsync(s->p, 0, pb, c->s) != hipSuccess ||
             hipMemsetAsync(s->count, 0, 64, c->s) != hipSuccess || hipMemsetAsync(s->stats, 0, 64, c->s) != hipSuccess) {
             surrogate_free(c);
@@ -990,7 +1026,7 @@ static SurrogateState* sstate(mhd_ctx* c) {
 void surrogate_free(mhd_ctx* c) {
     SurrogateState* s = c->sur;
     if (!s) return;
-    void* ps[] = {s->p, s->g, s->m, s->v, s->samples, s->count, s->scratch, s->loss, s->wbf, s->bias, s->stats,
+    void* ps[] = {s->p, s->m, s->v, s->samples, s->count, s->scratch, s->loss, s->wbf, s->bias, s->stats,
                   s->fix, s->net, s->ctr, s->blk};
     for (void* p : ps)
         if (p) hipFree(p);
@@ -1203,27 +1239,22 @@ int mhd_surrogate_fetch_samples(mhd_ctx* c, float* out, long n) {
     return sync_or(c);
 }
 
-// the minibatch scratch (activations and deltas of batch samples), then the
-// gradient's per-chunk partial sums
-static int ensure_scratch(mhd_ctx* c, SurrogateState* S, long batch) {
-    if (S->scratch_n >= batch) return MHD_OK;
-    if (S->scratch) hipFree(S->scratch);
-    S->scratch = nullptr;
-    S->scratch_n = 0;
-    const size_t n = (size_t)batch * sur::SC + (size_t)sur::kGradChunks * sur::NPARAM;
-    if (hipMalloc(&S->scratch, n * sizeof(float)) != hipSuccess) return MHD_ERR_HIP;
-    S->scratch_n = batch;
+// the gradient's per-chunk partial sums, then the chunks' squared errors
+static int ensure_scratch(SurrogateState* S) {
+    if (S->scratch) return MHD_OK;
+    const size_t n = (size_t)sur::kGradChunks * (sur::NPARAM + 1);
+    if (hipMalloc(&S->scratch, n * sizeof(float)) != hipSuccess) {
+        S->scratch = nullptr;
+        return MHD_ERR_HIP;
+    }
     return MHD_OK;
 }
+static float* loss_parts(SurrogateState* S) { return S->scratch + (size_t)sur::kGradChunks * sur::NPARAM; }
 
 static void run_minibatch(mhd_ctx* c, SurrogateState* S, const float* P, const float* set, long n, long first,
                           long mult, int batch) {
-    launch(c, MHD_K_SURR, blocks(batch), dim3(kBlock), sur::k_train_fb, P, set, n, first, mult, batch,
-           1.f / (float)(batch * sur::NO), S->scratch, S->loss);
-    float* gpart = S->scratch + (size_t)S->scratch_n * sur::SC;
-    launch(c, MHD_K_SURR, dim3((sur::NPARAM + 63) / 64, sur::kGradChunks / 4), dim3(kBlock), sur::k_train_grad,
-           (const float*)S->scratch, batch, gpart);
-    launch(c, MHD_K_SURR, dim3((sur::NPARAM + 255) / 256), dim3(256), sur::k_grad_sum, (const float*)gpart, S->g);
+    launch(c, MHD_K_SURR, dim3(sur::kGradChunks), dim3(sur::kTrainThreads), sur::k_train, P, set, n, first, mult,
+           batch, 1.f / (float)(batch * sur::NO), S->scratch, loss_parts(S));
 }
 
 static long gcd_l(long a, long b) {
@@ -1245,7 +1276,7 @@ int mhd_surrogate_train(mhd_ctx* c, int epochs, int batch, double lr, unsigned s
     if (hipStreamSynchronize(c->s) != hipSuccess) return MHD_ERR_HIP;
     n = n < S->cap ? n : S->cap;
     if (n < batch) return MHD_ERR_PARAM;
-    if (ensure_scratch(c, S, batch) != MHD_OK) return MHD_ERR_HIP;
+    if (ensure_scratch(S) != MHD_OK) return MHD_ERR_HIP;
     if (!S->have_weights) {  // deterministic initialisation: uniform(-1/sqrt(fan_in), 1/sqrt(fan_in))
         std::vector<float> w(sur::NPARAM, 0.f);
         unsigned long long z = 0x9E3779B97F4A7C15ull * (seed + 1);
@@ -1288,8 +1319,9 @@ int mhd_surrogate_train(mhd_ctx* c, int epochs, int batch, double lr, unsigned s
             const double b1c = 1. - std::pow(.9, (double)adam_t), b2c = 1. - std::pow(.999, (double)adam_t);
             const double prog = ((double)e + (double)bi / (double)nb) / (double)epochs;
             const double lr_t = lr * .5 * (1. + std::cos(3.141592653589793 * prog));
-            launch(c, MHD_K_SURR, dim3((sur::NPARAM + 255) / 256), dim3(256), sur::k_adam, S->p, S->g, S->m, S->v,
-                   (float)lr_t, (float)b1c, (float)b2c);
+            launch(c, MHD_K_SURR, dim3((sur::NPARAM + 63) / 64), dim3(64), sur::k_grad_adam,
+                   (const float*)S->scratch, (const float*)loss_parts(S), S->p, S->m, S->v, (float)lr_t, (float)b1c,
+                   (float)b2c, S->loss);
         }
         float h = 0.f;
         if (hipMemcpyAsync(&h, S->loss, sizeof(float), hipMemcpyDeviceToHost, c->s) != hipSuccess) return MHD_ERR_HIP;
@@ -1307,23 +1339,22 @@ int mhd_surrogate_grad(mhd_ctx* c, const float* w, const float* samples, int n, 
     hipSetDevice(c->p.device);
     SurrogateState* S = sstate(c);
     if (!S) return MHD_ERR_HIP;
-    if (ensure_scratch(c, S, n) != MHD_OK) return MHD_ERR_HIP;
-    // the given weights go to a buffer of their own: the context's net, its
-    // Adam moments and its gradient accumulator are left as they are
+    if (ensure_scratch(S) != MHD_OK) return MHD_ERR_HIP;
+    // the given weights go to a buffer of their own: the context's net and its
+    // Adam moments are left as they are
     float* dset = nullptr;
     if (hipMalloc(&dset, ((size_t)n * sur::NS + 2 * sur::NPARAM) * sizeof(float)) != hipSuccess) return MHD_ERR_HIP;
     float* dw = dset + (size_t)n * sur::NS;
     float* dg = dw + sur::NPARAM;
-    float* g_keep = S->g;
-    S->g = dg;
     int rc = MHD_OK;
     if (hipMemcpyAsync(dw, w, sur::NPARAM * sizeof(float), hipMemcpyHostToDevice, c->s) != hipSuccess ||
         hipMemcpyAsync(dset, samples, (size_t)n * sur::NS * sizeof(float), hipMemcpyHostToDevice, c->s) != hipSuccess)
         rc = MHD_ERR_HIP;
     if (rc == MHD_OK) {
         launch(c, MHD_K_SURR, dim3(1), dim3(64), sur::k_zero_f, S->loss, 1);
-        launch(c, MHD_K_SURR, dim3((sur::NPARAM + 255) / 256), dim3(256), sur::k_zero_f, dg, sur::NPARAM);
         run_minibatch(c, S, dw, dset, n, 0, 1, n);
+        launch(c, MHD_K_SURR, dim3((sur::NPARAM + 63) / 64), dim3(64), sur::k_grad_sum, (const float*)S->scratch,
+               (const float*)loss_parts(S), dg, S->loss);
         float h = 0.f;
         if (hipMemcpyAsync(grad, dg, sur::NPARAM * sizeof(float), hipMemcpyDeviceToHost, c->s) != hipSuccess ||
             hipMemcpyAsync(&h, S->loss, sizeof(float), hipMemcpyDeviceToHost, c->s) != hipSuccess)
@@ -1332,7 +1363,6 @@ int mhd_surrogate_grad(mhd_ctx* c, const float* w, const float* samples, int n, 
         if (rc == MHD_OK) rc = r2;
         if (loss) *loss = (double)h / (double)(n * sur::NO);
     }
-    S->g = g_keep;
     hipFree(dset);
     return rc;
 }
