@@ -23,10 +23,6 @@ namespace mhd {
 template <int M>
 struct VavFoot;
 template <>
-struct VavFoot<PDM> {
-    static constexpr int N = 8, LO = -4;
-};
-template <>
 struct VavFoot<TVD> {
     static constexpr int N = 4, LO = -2;
 };
@@ -92,27 +88,14 @@ struct VavWin {
     }
 };
 
-// PDM: the d1-interpolation of footprint column m2 (offset m2-4 along d2)
-template <typename R, bool MD1, bool U>
-__device__ __forceinline__ R pdm_col(const VavWin<R, PDM, MD1, U>& W, int m2) {
-    R s[8];
-#pragma unroll
-    for (int m1 = 0; m1 < 8; ++m1) s[m1] = W.cv(m1 - 4, m2 - 4);
-    return interp8(s);
-}
-
-// corner velocity of one edge from its window (mhd3d3.f90:1858-2116); for
-// PDM, g holds the 8 column interpolations (interp2_pdm's first sweep)
+// corner velocity of one edge from its window (mhd3d3.f90:1858-2116), TVD and
+// WENO.  (g holds nothing: without it in the marching loop the compiler writes
+// 2x as x+x in places of the fp32 MPWENO5 limiter, which then contract
+// differently, and the results are to stay what they are.)
 template <typename R, int M, bool MD1, bool U>
 __device__ __forceinline__ R vav_win(const VavWin<R, M, MD1, U>& W, const Coef<R>& c, const R* g = nullptr) {
     R v00_0, v10_0, v01_0, v11_0, v00_1, v01_1, v10_1, v11_1;
-    if constexpr (M == PDM) {
-        const R vi = interp8(g);
-        pdm2(W.cv(-2, -1), W.cv(-1, -1), W.cv(0, -1), W.cv(1, -1), vi, c.pdmb, v00_0, v10_0);
-        pdm2(W.cv(-1, -2), W.cv(-1, -1), W.cv(-1, 0), W.cv(-1, 1), vi, c.pdmb, v00_1, v01_1);
-        pdm2(W.cv(0, -2), W.cv(0, -1), W.cv(0, 0), W.cv(0, 1), vi, c.pdmb, v10_1, v11_1);
-        pdm2(W.cv(-2, 0), W.cv(-1, 0), W.cv(0, 0), W.cv(1, 0), vi, c.pdmb, v01_0, v11_0);
-    } else if constexpr (M == TVD) {
+    if constexpr (M == TVD) {
         const R vi = (W.cv(-1, -1) + W.cv(0, -1) + W.cv(0, 0) + W.cv(-1, 0)) / R(4);
         tvd(W.cv(-2, 0), W.cv(-1, 0), W.cv(0, 0), W.cv(1, 0), vi, c.eps, v00_0, v10_0);
         tvd(W.cv(0, -2), W.cv(0, -1), W.cv(0, 0), W.cv(0, 1), vi, c.eps, v00_1, v01_1);
@@ -167,11 +150,7 @@ __device__ __forceinline__ void step_fence(R& v) {
     __builtin_amdgcn_sched_barrier(0);
 }
 
-// corner velocities of T consecutive edges along the march axis
-// When the march runs along d2 (K=1, K=3), a step shifts the footprint by
-// one column, so seven of PDM's eight column interpolations carry over: they
-// ride along in a register window and only the new column is interpolated
-// (the same interp8 calls on the same values: bit-identical).
+// corner velocities of T consecutive edges along the march axis (TVD and WENO)
 template <typename R, int M, bool MD1, bool UNIT, int T, typename TI>
 __device__ __forceinline__ void vav_march(const TI* __restrict__ lv, ptrdiff_t b, ptrdiff_t s1, ptrdiff_t s2,
                                           const Coef<R>& c, R (&out)[T]) {
@@ -182,10 +161,6 @@ __device__ __forceinline__ void vav_march(const TI* __restrict__ lv, ptrdiff_t b
     VavWin<R, M, MD1, UNIT> W;
     W.load(lv, ob, osm, oso);
     R g[8];
-    if constexpr (M == PDM) {
-#pragma unroll
-        for (int m2 = 0; m2 < 8; ++m2) g[m2] = pdm_col(W, m2);
-    }
     // fp32 UNIT windows (the fewest registers): the next step's row is
     // loaded before the current corner velocity is computed, so its latency
     // hides behind that arithmetic (binary64 windows would lose a wave per
@@ -202,23 +177,12 @@ __device__ __forceinline__ void vav_march(const TI* __restrict__ lv, ptrdiff_t b
             ob += osm;
             if constexpr (PRE) W.shift_in(nxt);
             else W.shift(lv, ob, osm, oso);
-            if constexpr (M == PDM) {
-                if constexpr (MD1) {
-#pragma unroll
-                    for (int m2 = 0; m2 < 8; ++m2) g[m2] = pdm_col(W, m2);
-                } else {
-#pragma unroll
-                    for (int m2 = 0; m2 < 7; ++m2) g[m2] = g[m2 + 1];
-                    g[7] = pdm_col(W, 7);
-                }
-            }
         }
         step_fence(out[s]);
     };
-    // binary64 PDM (whose 8x8 window is 128 registers) and MPWENO5 run the
-    // steps as a loop: unrolled they need more registers than it saves
-    // (measured: 0.93 vs 0.66 ms for the binary64 ej march at 256^3)
-    if constexpr ((M == PDM && sizeof(R) == 8) || M == MPWENO5) {
+    // MPWENO5 runs the steps as a loop: unrolled they need more registers than
+    // it saves
+    if constexpr (M == MPWENO5) {
 #pragma unroll 1
         for (int s = 0; s < T; ++s) step(s);
     } else {
@@ -282,8 +246,8 @@ struct PdmLine {
 //     offset m-4; vi = interp8(g).  A step adds one row, so seven of the eight
 //     carry over.  Along d1 first, then d2 is interp2_pdm's order; for K=2
 //     (a = d1) that order holds only in fp32, which interpolates along d2 first
-//     (the same tensor-product value up to rounding); binary64 K=2 keeps the
-//     window march (vav_march) for bit parity.
+//     (the same tensor-product value up to rounding); binary64 K=2 shares its
+//     columns between lanes instead (pdm_columns, vav_march_cols).
 //   * the four PDM2 lines: two across the march (along b, at a = -1 and 0) and
 //     two along it (along a, at b = -1 and 0); a step hands the a = 0 line on
 //     as the next a = -1 one and slides the other two (PdmLine).
@@ -380,6 +344,85 @@ __device__ __forceinline__ void vav_march_pdm(const TI* __restrict__ lv, const B
     }
 }
 
+// Binary64 ej (K=2, corner plane (z, x), march along z).  interp2_pdm's order
+// interpolates along z first: the eight columns x-4..x+3 of the footprint at every
+// edge.  A column is the same for the eight edges along x that it serves, and
+// lanes run along x, so each lane interpolates its own column (pdm_columns: one
+// load and one interpolation per step and velocity) and the lanes exchange the
+// results through LDS.  Lanes stand for columns here: a row of ii edges has
+// ii + 7, and a workgroup's outer 4 + 3 only interpolate.  An 8x8 window per lane
+// interpolated eight columns per step and needed 206 registers: the three
+// directions took 1.49 ms at 256^3, 1.22 ms with this; a 64^3 step 228 and 208 us.
+// Bound: VALU issue, at 3 wavefronts per SIMD (160 registers).
+constexpr int kColEdges = kBlock - 7;
+template <typename R, int T, typename TI>
+__device__ __forceinline__ void pdm_columns(const Buf<TI>& bv, unsigned ob, unsigned osm, R (*cols)[kBlock]) {
+    const unsigned o0 = ob - 4u * osm;
+    R w[8];
+#pragma unroll
+    for (int m = 0; m < 8; ++m) w[m] = R(bv.at(o0, (unsigned)m * osm));
+#pragma unroll
+    for (int s = 0; s < T; ++s) {
+        cols[s][threadIdx.x] = interp8(w);
+        if (s + 1 < T) {
+#pragma unroll
+            for (int m = 0; m < 7; ++m) w[m] = w[m + 1];
+            w[7] = R(bv.at(o0, (unsigned)(s + 8) * osm));
+        }
+    }
+}
+
+// the march's corner velocities from the lanes' columns: V[a+2][b+2] holds the
+// footprint's core, a = -2..1 along z, b = -2..1 along x (see vav_march_pdm)
+template <typename R, int T, typename TI>
+__device__ __forceinline__ void vav_march_cols(const TI* __restrict__ lv, unsigned ob, unsigned osm, const Coef<R>& c,
+                                               const R (*cols)[kBlock], R (&out)[T]) {
+    auto row = [&](unsigned orow, R* v) {
+        const TI* p = reinterpret_cast<const TI*>(reinterpret_cast<const char*>(lv) + orow);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) v[q] = R(p[q - 2]);
+    };
+    const R pdmb = c.pdmb;
+    R V[4][4];
+#pragma unroll
+    for (int a = 0; a < 4; ++a) row(ob + (unsigned)(a - 2) * osm, V[a]);
+    PdmLine<R> C0, C1, L0, L1;
+    C0.set(V[1][0], V[1][1], V[1][2], V[1][3], pdmb);
+    C1.set(V[2][0], V[2][1], V[2][2], V[2][3], pdmb);
+    L0.set(V[0][1], V[1][1], V[2][1], V[3][1], pdmb);
+    L1.set(V[0][2], V[1][2], V[2][2], V[3][2], pdmb);
+#pragma unroll
+    for (int s = 0; s < T; ++s) {
+        R g[8];
+#pragma unroll
+        for (int m = 0; m < 8; ++m) g[m] = cols[s][(int)threadIdx.x + m - 4];
+        const R vi = interp8(g);
+        auto cv = [&](int o1, int o2) { return V[o1 + 2][o2 + 2]; };
+        R v00_0, v10_0, v00_1, v01_1, v10_1, v11_1, v01_0, v11_0;
+        L0.finish(cv(-1, -1), cv(0, -1), vi, v00_0, v10_0);
+        C0.finish(cv(-1, -1), cv(-1, 0), vi, v00_1, v01_1);
+        C1.finish(cv(0, -1), cv(0, 0), vi, v10_1, v11_1);
+        L1.finish(cv(-1, 0), cv(0, 0), vi, v01_0, v11_0);
+        const R v00 = pick(sgn1(fabs(L0.rm) - fabs(C0.rm)), v00_0, v00_1);
+        const R v10 = pick(sgn1(fabs(L0.rp) - fabs(C1.rm)), v10_0, v10_1);
+        const R v01 = pick(sgn1(fabs(L1.rm) - fabs(C0.rp)), v01_0, v01_1);
+        const R v11 = pick(sgn1(fabs(L1.rp) - fabs(C1.rp)), v11_0, v11_1);
+        out[s] = R(.25) * (v00 + v01 + v10 + v11);
+        if (s + 1 < T) {
+#pragma unroll
+            for (int a = 0; a < 3; ++a)
+#pragma unroll
+                for (int b = 0; b < 4; ++b) V[a][b] = V[a + 1][b];
+            row(ob + (unsigned)(s + 2) * osm, V[3]);
+            C0 = C1;
+            C1.set(V[2][0], V[2][1], V[2][2], V[2][3], pdmb);
+            L0.slide(V[1][1], V[2][1], V[3][1], pdmb);
+            L1.slide(V[1][2], V[2][2], V[3][2], pdmb);
+        }
+        step_fence(out[s]);
+    }
+}
+
 // workgroups of the ei march: 64 x-lanes by 4 consecutive y edges, one run
 // of T edges along z
 template <int T>
@@ -401,7 +444,8 @@ struct EmfGeom {
 };
 
 // threads = ii * no * ceil(nm / T) (K=2, 3) or emf_tiles workgroups (K=1);
-// lanes run along x
+// lanes run along x.  Binary64 PDM's ej: threads = (ii + 7) * no * ceil(nm / T)
+// columns, kColEdges of them a workgroup's own
 template <typename R, int M, int K, int T, typename TI, typename TF>
 __global__ void __launch_bounds__(kBlock) k_emf_march(Dims d, Coef<R> c, EmfIn<TI> in, R ef,
                                                      const double* __restrict__ efa, TF* __restrict__ e,

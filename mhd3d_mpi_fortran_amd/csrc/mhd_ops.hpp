@@ -119,14 +119,27 @@ void flux_launch(mhd_ctx* c, Src<TI> s) {
     }
 }
 
+// threads and workgroups of direction K's march (k_emf_march)
+template <typename R, int M, int K, int T>
+long emf_threads(const Dims& d) {
+    const long ii = d.nx0 + (K != 1) + (M == PDM && K == 2 && sizeof(R) == 8 ? 7 : 0);
+    const long no = K == 3 ? d.nz0 : (K == 1 ? d.ny0 + 1 : d.ny0);
+    const long nm = K == 3 ? d.ny0 + 1 : d.nz0 + 1;
+    return ii * no * ((nm + T - 1) / T);
+}
+template <typename R, int M, int K, int T>
+unsigned emf_blocks(const Dims& d) {
+    if (K == 1) return emf_tiles<T>(d.nx0, d.ny0, d.nz0);
+    const long n = emf_threads<R, M, K, T>(d);
+    if (M == PDM && K == 2 && sizeof(R) == 8) return (unsigned)((n + kColEdges - 1) / kColEdges);
+    return blocks(n).x;
+}
+
 template <typename R, int M, int K, int T, typename TI, typename TF>
 void emf_launch_kt(mhd_ctx* c, EmfIn<TI> in) {
     const Dims& d = c->d;
-    const long ii = d.nx0 + (K != 1);
-    const long no = K == 3 ? d.nz0 : (K == 1 ? d.ny0 + 1 : d.ny0);
-    const long nm = K == 3 ? d.ny0 + 1 : d.nz0 + 1;
-    const long n = ii * no * ((nm + T - 1) / T);
-    const dim3 grid = K == 1 ? dim3(emf_tiles<T>(d.nx0, d.ny0, d.nz0)) : blocks(n);
+    const long n = emf_threads<R, M, K, T>(d);
+    const dim3 grid(emf_blocks<R, M, K, T>(d));
     launch(c, MHD_K_EMF, grid, dim3(kBlock), k_emf_march<R, M, K, T, TI, TF>, d, make_coef<R>(c), in,
            R(c->met.ef[K - 1]), c->met.mode == 2 ? c->gm.ef[K - 1] : (const double*)nullptr, (TF*)c->emf[K - 1], n);
 }
@@ -221,12 +234,12 @@ void stage_launch_mm(mhd_ctx* c, Src<TI> s, int what) {
         o.efa[a] = c->met.mode == 2 ? c->gm.ef[a] : nullptr;
     }
     if ((what & kStageEmf) && march) {
-        for (int a = 0; a < 3; ++a) {
-            const long ii = d.nx0 + (a != 0), no = a == 2 ? d.nz0 : (a == 0 ? d.ny0 + 1 : d.ny0);
-            const long nm = a == 2 ? d.ny0 + 1 : d.nz0 + 1;
-            o.nthreads[a] = ii * no * ((nm + T - 1) / T);
-            nb[a] = a == 0 ? emf_tiles<T>(d.nx0, d.ny0, d.nz0) : blocks(o.nthreads[a]).x;
-        }
+        o.nthreads[0] = emf_threads<R, M, 1, T>(d);
+        o.nthreads[1] = emf_threads<R, M, 2, T>(d);
+        o.nthreads[2] = emf_threads<R, M, 3, T>(d);
+        nb[0] = emf_blocks<R, M, 1, T>(d);
+        nb[1] = emf_blocks<R, M, 2, T>(d);
+        nb[2] = emf_blocks<R, M, 3, T>(d);
     }
     if (what & kStageFlux) {
         nb[3] = face_tiles<2>(d.nx0, d.ny0 + 1, d.nz0);
