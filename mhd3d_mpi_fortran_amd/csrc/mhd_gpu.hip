@@ -822,6 +822,24 @@ static void do_ct_t(mhd_ctx* c, double* const* out) {
            (const double*)c->dy, (const double*)c->dz, gmet(c));
 }
 
+// the cell update and CT in one launch (k_advance)
+template <typename TF, int NST, int ST>
+static void do_advance_t(mhd_ctx* c, double* const* out) {
+    const CCells s{c->rho, c->vx, c->vy, c->vz, c->pr};
+    const Cells so{out[0], out[1], out[2], out[3], out[4]};
+    const PrevRK pv{c->rhop, c->mxp, c->myp, c->mzp, c->engp};
+    const FluxSet<TF> F{(const TF*)c->flux[0], (const TF*)c->flux[1], (const TF*)c->flux[2],
+                        c->nf[0], c->nf[1], c->nf[2]};
+    const unsigned nupd = blocks(c->ninterior).x;
+    auto k = c->met.mode == 2 ? k_advance<NST, ST, TF, true> : k_advance<NST, ST, TF, false>;
+    launch(c, MHD_K_UPDATE, dim3(nupd + blocks(c->nf[0] + c->nf[1] + c->nf[2]).x), dim3(kBlock), k, c->d,
+           c->p.gam - 1., (const double*)(c->scal + SC_TAU), s, so, pv, F, sdx(c), sdy(c), sdz(c), gmet(c),
+           c->ninterior, nupd, CtFactor{{c->met.ct[0], c->met.ct[1], c->met.ct[2]}}, CFaces{c->bi, c->bj, c->bk},
+           Faces{out[8], out[9], out[10]}, Faces{c->bip, c->bjp, c->bkp}, (const TF*)c->emf[0],
+           (const TF*)c->emf[1], (const TF*)c->emf[2], (const double*)c->dx, (const double*)c->dy,
+           (const double*)c->dz);
+}
+
 // One stage's stencil work and update on two streams.  The edge EMF and,
 // behind it, the CT face update run on the second stream; the face flux and
 // the cell update on the main stream.  The EMF reads the stage's
@@ -856,9 +874,16 @@ static void stage_overlapped(mhd_ctx* c, E emf, F flux, B both, double* const* o
             emf();
             flux();
         }
-        if (after_ct) ct();
-        cells();
-        if (!after_ct) ct();
+        if (after_ct) {
+            ct();
+            cells();
+        } else if (c->merged) {
+            if (mixed(c)) do_advance_t<float, NST, ST>(c, out);
+            else do_advance_t<double, NST, ST>(c, out);
+        } else {
+            cells();
+            ct();
+        }
         return;
     }
     c->cur = c->s2;
@@ -1293,9 +1318,17 @@ static void advance_serial(mhd_ctx* c) {
     double* self[11];
     for (int a = 0; a < 11; ++a) self[a] = *state_slot(c, a);
     if (mixed(c)) {
+        if (c->merged) {
+            do_advance_t<float, NST, ST>(c, self);
+            return;
+        }
         do_cells_t<float, NST, ST>(c, self, false);
         do_ct_t<float, NST, ST>(c, self);
     } else {
+        if (c->merged) {
+            do_advance_t<double, NST, ST>(c, self);
+            return;
+        }
         do_cells_t<double, NST, ST>(c, self, false);
         do_ct_t<double, NST, ST>(c, self);
     }
