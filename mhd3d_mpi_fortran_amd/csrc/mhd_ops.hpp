@@ -45,7 +45,7 @@ struct StencilOut {
     long nthreads[3];      // EMF threads per direction
     unsigned end[6];       // last workgroup + 1 of the EMF's and the flux's directions
 };
-template <typename R, int M, typename TI, typename TF, int MET, bool EMF>
+template <typename R, int M, typename TI, typename TF, int MET, bool EMF, int T>
 __global__ void __launch_bounds__(kBlock) k_stencils(Dims d, Coef<R> c, Prim<TI> q, Normals<R> nm, GMet gm,
                                                     EmfIn<TI> e1, EmfIn<TI> e2, EmfIn<TI> e3,
                                                     StencilOut<R, TF> o) {
@@ -55,7 +55,6 @@ __global__ void __launch_bounds__(kBlock) k_stencils(Dims d, Coef<R> c, Prim<TI>
         const unsigned lo = p ? o.end[p - 1] : 0;
         return xcd_map(b - lo, o.end[p] - lo);
     };
-    constexpr int T = EmfSteps<M, 1>::T_SHORT;
     if constexpr (EMF) {
         if (b < o.end[0]) {
             emf_block<R, M, 1, T, TI, TF>(d, c, e1, o.ef[0], o.efa[0], o.emf[0], o.nthreads[0], place(0));
@@ -219,11 +218,10 @@ void emf_launch(mhd_ctx* c, Src<TI> s) {
 }
 
 // a stage's stencils in one launch (what: kStageFlux | kStageEmf)
-template <typename R, typename TI, typename TF, int M, int MET>
-void stage_launch_mm(mhd_ctx* c, Src<TI> s, int what) {
+template <typename R, typename TI, typename TF, int M, int MET, int T>
+void stage_launch_t(mhd_ctx* c, Src<TI> s, int what) {
     const Dims& d = c->d;
     constexpr bool march = M == PDM || M == TVD;
-    constexpr int T = EmfSteps<M, 1>::T_SHORT;
     StencilOut<R, TF> o{};
     unsigned nb[6] = {0, 0, 0, 0, 0, 0};
     for (int a = 0; a < 3; ++a) {
@@ -252,12 +250,35 @@ void stage_launch_mm(mhd_ctx* c, Src<TI> s, int what) {
     const TI* u[3] = {s.vx, s.vy, s.vz};
     if (c->met.on)
         for (int a = 0; a < 3; ++a) u[a] = s.w[a];
-    launch(c, what & kStageFlux ? MHD_K_FLUX : MHD_K_EMF, dim3(n), dim3(kBlock), k_stencils<R, M, TI, TF, MET, march>, d,
+    launch(c, what & kStageFlux ? MHD_K_FLUX : MHD_K_EMF, dim3(n), dim3(kBlock), k_stencils<R, M, TI, TF, MET, march, T>, d,
            make_coef<R>(c), q, make_normals<R>(c), c->gm, EmfIn<TI>{u[1], u[2], s.bj, s.bk, s.vf},
            EmfIn<TI>{u[2], u[0], s.bk, s.bi, s.vf}, EmfIn<TI>{u[0], u[1], s.bi, s.bj, s.vf}, o);
     if constexpr (!march) {
         if (what & kStageEmf) emf_launch_m<R, TI, TF, M>(c, s);
     }
+}
+
+// EMF runs of 2 edges per thread; binary64 PDM, whose run start (an 8x8 footprint)
+// costs most, takes runs of 4 once runs of 2 give the stage more workgroups than
+// there are CUs: below that a stage lasts as long as its longest thread
+// (16^3: 44 us a step with runs of 2, 56 with 4, 80 with 8), above as long
+// as its arithmetic (24^3: 53 and 52 us; 64^3: 191 and 181; 96^3: 641 and 605; runs
+// of 8, at two wavefronts per SIMD, 67, 192 and 642).  TVD's starts are cheap (96^3:
+// 566 and 561 us, 32^3: 60 and 61) and fp32 results may depend on the place in a run.
+template <typename R, typename TI, typename TF, int M, int MET>
+void stage_launch_mm(mhd_ctx* c, Src<TI> s, int what) {
+    constexpr int T = EmfSteps<M, 1>::T_SHORT;
+    const Dims& d = c->d;
+    if constexpr (M == PDM && sizeof(R) == 8) {
+        const unsigned n = emf_blocks<R, M, 1, T>(d) + emf_blocks<R, M, 2, T>(d) + emf_blocks<R, M, 3, T>(d) +
+                           face_tiles<2>(d.nx0, d.ny0 + 1, d.nz0) + face_tiles<3>(d.nx0, d.ny0, d.nz0 + 1) +
+                           blocks(c->nf[0]).x;
+        if (n > 256) {
+            stage_launch_t<R, TI, TF, M, MET, 4>(c, s, what);
+            return;
+        }
+    }
+    stage_launch_t<R, TI, TF, M, MET, T>(c, s, what);
 }
 
 template <typename R, typename TI, typename TF, int M>
