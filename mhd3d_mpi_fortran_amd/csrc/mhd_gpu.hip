@@ -217,6 +217,12 @@ int mhd_create(mhd_ctx** out, const mhd_params* p) {
         mhd_destroy(c);
         return MHD_ERR_HIP;
     }
+    if (hipHostMalloc(&c->hscal, 4 * sizeof(double), hipHostMallocDefault) != hipSuccess) {
+        c->hscal = nullptr;
+        mhd_destroy(c);
+        return MHD_ERR_HIP;
+    }
+    c->hscal[0] = c->hscal[1] = 0.;
     // zero everything once so ghost shells and unused slots hold defined values
     if (hipMemsetAsync(c->arena, 0, state, c->s) != hipSuccess || hipStreamSynchronize(c->s) != hipSuccess) {
         mhd_destroy(c);
@@ -240,6 +246,7 @@ void mhd_destroy(mhd_ctx* c) {
     if (c->metbuf) hipFree(c->metbuf);
     if (c->gmetbuf) hipFree(c->gmetbuf);
     if (c->arena) hipFree(c->arena);
+    if (c->hscal) hipHostFree(c->hscal);
     if (c->ev_fork) hipEventDestroy(c->ev_fork);
     if (c->ev_join) hipEventDestroy(c->ev_join);
     if (c->ev_emf) hipEventDestroy(c->ev_emf);
@@ -762,7 +769,8 @@ static void do_bxyz(mhd_ctx* c, bool want_vf, bool want_shadow, bool want_dt, bo
 // get_dt on the current state; the minimum lands in scal[SC_DTCFL] and, when
 // set_tau, also in scal[SC_TAU] (Adams-Bashforth takes tau from the CFL);
 // fixed != null: tau = tau0 = *fixed instead (Runge-Kutta)
-static void do_dt(mhd_ctx* c, bool set_tau, const double* fixed = nullptr) {
+// `report`: the call returns them, k_dt_final writes c->hscal too
+static void do_dt(mhd_ctx* c, bool set_tau, const double* fixed = nullptr, bool report = false) {
     // where cell B of the current state is not stored (mixed Adams-Bashforth
     // steps, uploads), get_bxyz forms it and the CFL partials in one pass
     if (!c->dt_fresh && c->cellb_stale) do_bxyz(c, false, false, true);
@@ -773,7 +781,8 @@ static void do_dt(mhd_ctx* c, bool set_tau, const double* fixed = nullptr) {
         n = blocks(c->ncell).x;
     }
     launch(c, MHD_K_DT, dim3(1), dim3(1024), k_dt_final, (const double*)c->dtpart, n, c->scal + SC_DTCFL,
-           set_tau || fixed ? c->scal + SC_TAU : (double*)nullptr, fixed ? 1 : 0, fixed ? *fixed : 0.);
+           set_tau || fixed ? c->scal + SC_TAU : (double*)nullptr, fixed ? 1 : 0, fixed ? *fixed : 0.,
+           report ? c->hscal : (double*)nullptr);
 }
 
 // conserved update from the current state into `out` (the current state
@@ -1002,12 +1011,9 @@ int mhd_get_bxyz(mhd_ctx* c) {
 int mhd_get_dt(mhd_ctx* c, double* tau_cfl) {
     if (!c || !c->have_geometry) return MHD_ERR_PARAM;
     hipSetDevice(c->p.device);
-    do_dt(c, true);   // get_dt sets the module's tau (mhd3d3.f90:1629)
-    double h = 0.;
-    if (hipMemcpyAsync(&h, c->scal + SC_DTCFL, sizeof(double), hipMemcpyDeviceToHost, c->s) != hipSuccess)
-        return MHD_ERR_HIP;
-    int rc = sync_status(c);
-    if (tau_cfl) *tau_cfl = h;
+    do_dt(c, true, nullptr, true);   // get_dt sets the module's tau (mhd3d3.f90:1629)
+    const int rc = sync_status(c);
+    if (tau_cfl) *tau_cfl = rc == MHD_OK ? c->hscal[1] : 0.;
     return rc;
 }
 
@@ -1178,8 +1184,8 @@ int mhd_initialize(mhd_ctx* c, double* tau) {
 
 // step_rk2 / step_rk3 (mhd3d3.f90:3648-3792), in place
 template <int NST>
-static void step_rk(mhd_ctx* c) {
-    do_dt(c, false, &c->tau0_host);
+static void step_rk(mhd_ctx* c, bool report = false) {
+    do_dt(c, false, &c->tau0_host, report);
     double* self[11];
     for (int a = 0; a < 11; ++a) self[a] = *state_slot(c, a);
     for (int st = 1; st <= NST; ++st) {
@@ -1228,8 +1234,8 @@ static void predict_ab(mhd_ctx* c) {
     }
 }
 
-static void step_ab(mhd_ctx* c) {
-    do_dt(c, true);
+static void step_ab(mhd_ctx* c, bool report) {
+    do_dt(c, true, nullptr, report);
     predict_ab(c);
     const bool fused = can_fuse(c);
     if (fused) stage_fused(c, c->xn);
@@ -1257,14 +1263,19 @@ int mhd_step(mhd_ctx* c, int nsteps, double* tau, double* tau_cfl) {
     if (c->p.stepop != 1 && tau) c->tau0_host = *tau;
     if (nsteps > 0) c->pred_valid = false;
     for (int n = 0; n < nsteps; ++n) {
-        if (c->p.stepop == 1) step_ab(c);
-        else if (c->p.stepop == 2) step_rk<2>(c);
-        else step_rk<3>(c);
+        const bool report = n == nsteps - 1;
+        if (c->p.stepop == 1) step_ab(c, report);
+        else if (c->p.stepop == 2) step_rk<2>(c, report);
+        else step_rk<3>(c, report);
     }
     double h[3] = {0., 0., 0.};
-    if (hipMemcpyAsync(h, c->scal, 3 * sizeof(double), hipMemcpyDeviceToHost, c->s) != hipSuccess)
+    if (nsteps == 0 && hipMemcpyAsync(h, c->scal, 3 * sizeof(double), hipMemcpyDeviceToHost, c->s) != hipSuccess)
         return MHD_ERR_HIP;
-    int rc = sync_status(c);
+    const int rc = sync_status(c);
+    if (nsteps > 0) {
+        h[SC_TAU] = c->hscal[0];
+        h[SC_DTCFL] = c->hscal[1];
+    }
     if (tau) *tau = h[SC_TAU];
     if (tau_cfl) *tau_cfl = h[SC_DTCFL];
     return rc;
@@ -1615,7 +1626,7 @@ int mhd_divb_max(mhd_ctx* c, double* divb) {
     launch(c, MHD_K_DT, g, dim3(kBlock), k, c->d, CFaces{c->bi, c->bj, c->bk}, sdx(c), sdy(c), sdz(c), gmet(c),
            c->divpart, c->ninterior);
     launch(c, MHD_K_DT, dim3(1), dim3(1024), k_dt_final, (const double*)c->divpart, (long)g.x, c->scal + SC_DIVB,
-           (double*)nullptr, 0, 0.);
+           (double*)nullptr, 0, 0., (double*)nullptr);
     double h = 0.;
     if (hipMemcpyAsync(&h, c->scal + SC_DIVB, sizeof(double), hipMemcpyDeviceToHost, c->s) != hipSuccess)
         return MHD_ERR_HIP;

@@ -109,6 +109,7 @@ struct mhd_ctx {
     double* divpart = nullptr;   // per-workgroup partials of the div B monitor (apart from the CFL ones)
     double* scal = nullptr;
     int* flags = nullptr;
+    double* hscal = nullptr;   // pinned: tau and the CFL minimum of the last step of a call (k_dt_final)
     double tau0_host = 0.;
     hipError_t launch_error = hipSuccess;
     // kernel timing
