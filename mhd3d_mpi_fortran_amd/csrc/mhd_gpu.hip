@@ -822,11 +822,9 @@ static void do_ct_t(mhd_ctx* c, double* const* out) {
     CFaces b{c->bi, c->bj, c->bk};
     Faces bo{out[8], out[9], out[10]};
     Faces bp{c->bip, c->bjp, c->bkp};
-    const long nct = (long)(c->d.nx0 + 1) * c->d.ny0 * c->d.nz0 + (long)c->d.nx0 * (c->d.ny0 + 1) * c->d.nz0 +
-                     (long)c->d.nx0 * c->d.ny0 * (c->d.nz0 + 1);
     const CtFactor ctf{{c->met.ct[0], c->met.ct[1], c->met.ct[2]}};
     auto kc = c->met.mode == 2 ? k_ct<NST, ST, TF, true> : k_ct<NST, ST, TF, false>;
-    launch(c, MHD_K_CT, blocks(nct), dim3(kBlock), kc, c->d, (const double*)(c->scal + SC_TAU), ctf, b,
+    launch(c, MHD_K_CT, blocks(ct_corners(c->d)), dim3(kBlock), kc, c->d, (const double*)(c->scal + SC_TAU), ctf, b,
            bo, bp, (const TF*)c->emf[0], (const TF*)c->emf[1], (const TF*)c->emf[2], (const double*)c->dx,
            (const double*)c->dy, (const double*)c->dz, gmet(c));
 }
@@ -841,7 +839,7 @@ static void do_advance_t(mhd_ctx* c, double* const* out) {
                         c->nf[0], c->nf[1], c->nf[2]};
     const unsigned nupd = blocks(c->ninterior).x;
     auto k = c->met.mode == 2 ? k_advance<NST, ST, TF, true> : k_advance<NST, ST, TF, false>;
-    launch(c, MHD_K_UPDATE, dim3(nupd + blocks(c->nf[0] + c->nf[1] + c->nf[2]).x), dim3(kBlock), k, c->d,
+    launch(c, MHD_K_UPDATE, dim3(nupd + blocks(ct_corners(c->d)).x), dim3(kBlock), k, c->d,
            c->p.gam - 1., (const double*)(c->scal + SC_TAU), s, so, pv, F, sdx(c), sdy(c), sdz(c), gmet(c),
            c->ninterior, nupd, CtFactor{{c->met.ct[0], c->met.ct[1], c->met.ct[2]}}, CFaces{c->bi, c->bj, c->bk},
            Faces{out[8], out[9], out[10]}, Faces{c->bip, c->bjp, c->bkp}, (const TF*)c->emf[0],
