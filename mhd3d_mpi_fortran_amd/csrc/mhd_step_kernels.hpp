@@ -755,7 +755,7 @@ __global__ void __launch_bounds__(kBlock) k_predict_ab_mixed(Dims d, AB11<float>
                                                             const double* __restrict__ tau_p,
                                                             float* __restrict__ vfh, Proj<float> pj, long ncell,
                                                             long nbi, long nbj, long nbk) {
-    const long t = gtid_xcd();
+    const long t = gtid_plane((unsigned)d.nx * (unsigned)d.ny);
     const double c = tau_p[0] / tau_p[1] / 2.;
     auto ext = [&](const double* x, const double* xp, ptrdiff_t f) { return x[f] + c * (x[f] - xp[f]); };
     if (t < ncell) {
