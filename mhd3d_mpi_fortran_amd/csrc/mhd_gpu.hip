@@ -16,6 +16,7 @@
 #include <vector>
 
 #include "mhd_fused.hpp"
+#include "mhd_sweep_args.hpp"
 #include "mhd_launch.hpp"
 #include "mhd_step_kernels.hpp"
 
@@ -785,6 +786,27 @@ static void do_dt(mhd_ctx* c, bool set_tau, const double* fixed = nullptr, bool 
            report ? c->hscal : (double*)nullptr);
 }
 
+// a binary64 Adams-Bashforth stage's z fluxes and update in one kernel
+// (mhd_sweep.hpp); Runge-Kutta updates in place the cells whose neighbours'
+// fluxes are still to be formed
+static bool can_sweep(const mhd_ctx* c) {
+    return !mixed(c) && c->p.stepop == 1 && !c->merged && !c->p.surrogate && c->met.mode != 2;
+}
+static SweepArgs sweep_args(const mhd_ctx* c, double* const* out, bool keep) {
+    SweepArgs a{};
+    a.F = FluxSet<double>{(const double*)c->flux[0], (const double*)c->flux[1], nullptr, c->nf[0], c->nf[1], c->nf[2]};
+    a.fz = keep ? (double*)c->flux[2] : nullptr;
+    a.gm1 = c->p.gam - 1.;
+    a.tau_p = c->scal + SC_TAU;
+    a.s = CCells{c->rho, c->vx, c->vy, c->vz, c->pr};
+    a.so = Cells{out[0], out[1], out[2], out[3], out[4]};
+    a.dx = sdx(c);
+    a.dy = sdy(c);
+    a.dz = sdz(c);
+    a.cells = sweep_cells(c->d);
+    return a;
+}
+
 // conserved update from the current state into `out` (the current state
 // itself for RK, the next-state buffers for AB)
 template <typename TF, int NST, int ST>
@@ -966,6 +988,24 @@ static void stage_fused(mhd_ctx* c, double* const* out) {
     if (dt) hipStreamWaitEvent(c->s, c->ev_join, 0);
     launch_flux_update(c, a, dt);
     if (!dt) hipStreamWaitEvent(c->s, c->ev_join, 0);
+}
+
+// such a stage: EMF and CT beside the x and y fluxes and the sweep, which write
+// buffers of their own.  keep: the z fluxes are left in memory too
+static void stage_sweep(mhd_ctx* c, double* const* out, bool keep) {
+    const Src<double> h = h_src(c);
+    const bool ok = c->overlap && hipEventRecord(c->ev_fork, c->s) == hipSuccess &&
+                    hipStreamWaitEvent(c->s2, c->ev_fork, 0) == hipSuccess;
+    if (ok) c->cur = c->s2;
+    launch_emf_fp64(c, h);
+    do_ct_t<double, 0, 0>(c, out);
+    if (ok) {
+        hipEventRecord(c->ev_join, c->s2);
+        c->cur = nullptr;
+    }
+    launch_flux_fp64(c, h, false);
+    launch_sweep_fp64(c, h, sweep_args(c, out, keep));
+    if (ok) hipStreamWaitEvent(c->s, c->ev_join, 0);
 }
 
 template <int NST, int ST>
@@ -1237,6 +1277,7 @@ static void step_ab(mhd_ctx* c, bool report) {
     predict_ab(c);
     const bool fused = can_fuse(c);
     if (fused) stage_fused(c, c->xn);
+    else if (can_sweep(c)) stage_sweep(c, c->xn, report);
     else do_stage<0, 0>(c, h_src(c), c->xn);
     // rotate: previous <- current <- next <- previous
     for (int a = 0; a < 11; ++a) {

@@ -202,7 +202,8 @@ inline mhd::Normals<R> make_normals(const mhd_ctx* c) {
 }
 
 // per-precision stencil launchers (separate translation units)
-void launch_flux_fp64(mhd_ctx* c, mhd::Src<double> s);
+// z: the z faces too (false: a sweep forms them, mhd_sweep.hpp)
+void launch_flux_fp64(mhd_ctx* c, mhd::Src<double> s, bool z = true);
 void launch_emf_fp64(mhd_ctx* c, mhd::Src<double> s);
 void launch_recon(mhd_ctx* c, int dir, const double* f, int fn1, int fn2, int lnx, int lny, int lnz, double* fl,
                   double* fr);

@@ -75,7 +75,7 @@ __global__ void __launch_bounds__(kBlock) k_stencils(Dims d, Coef<R> c, Prim<TI>
 }
 
 template <typename R, typename TI, typename TF, int M, int MET>
-void flux_launch_mm(mhd_ctx* c, Src<TI> s) {
+void flux_launch_mm(mhd_ctx* c, Src<TI> s, bool z) {
     const Coef<R> co = make_coef<R>(c);
     const Prim<TI> q{s.rho, s.vx, s.vy, s.vz, s.p, s.bx, s.by, s.bz};
     const Normals<R> nm = make_normals<R>(c);
@@ -93,6 +93,7 @@ void flux_launch_mm(mhd_ctx* c, Src<TI> s) {
     else
         launch(c, MHD_K_FLUX, dim3(face_tiles<2>(d.nx0, d.ny0 + 1, d.nz0)), dim3(kBlock),
                k_flux<R, M, 2, TI, TF, MET>, c->d, co, q, nm, c->gm, (TF*)c->flux[1], c->nf[1]);
+    if (!z) return;
     if (fp32 && z8 >= (unsigned)kFluxRunBlocks)
         launch(c, MHD_K_FLUX, dim3(z8), dim3(kBlock), k_flux<R, M, 3, TI, TF, MET, kFluxRun>, c->d, co, q, nm,
                c->gm, (TF*)c->flux[2], c->nf[2]);
@@ -102,19 +103,19 @@ void flux_launch_mm(mhd_ctx* c, Src<TI> s) {
 }
 
 template <typename R, typename TI, typename TF, int M>
-void flux_launch_m(mhd_ctx* c, Src<TI> s) {
-    if (c->met.mode == 2) flux_launch_mm<R, TI, TF, M, 2>(c, s);
-    else if (c->met.on) flux_launch_mm<R, TI, TF, M, 1>(c, s);
-    else flux_launch_mm<R, TI, TF, M, 0>(c, s);
+void flux_launch_m(mhd_ctx* c, Src<TI> s, bool z) {
+    if (c->met.mode == 2) flux_launch_mm<R, TI, TF, M, 2>(c, s, z);
+    else if (c->met.on) flux_launch_mm<R, TI, TF, M, 1>(c, s, z);
+    else flux_launch_mm<R, TI, TF, M, 0>(c, s, z);
 }
 
 template <typename R, typename TI, typename TF>
-void flux_launch(mhd_ctx* c, Src<TI> s) {
+void flux_launch(mhd_ctx* c, Src<TI> s, bool z) {
     switch (c->p.reconop) {
-    case PDM: flux_launch_m<R, TI, TF, PDM>(c, s); break;
-    case TVD: flux_launch_m<R, TI, TF, TVD>(c, s); break;
-    case WENO5: flux_launch_m<R, TI, TF, WENO5>(c, s); break;
-    default: flux_launch_m<R, TI, TF, MPWENO5>(c, s); break;
+    case PDM: flux_launch_m<R, TI, TF, PDM>(c, s, z); break;
+    case TVD: flux_launch_m<R, TI, TF, TVD>(c, s, z); break;
+    case WENO5: flux_launch_m<R, TI, TF, WENO5>(c, s, z); break;
+    default: flux_launch_m<R, TI, TF, MPWENO5>(c, s, z); break;
     }
 }
 

@@ -10,7 +10,7 @@ void launch_stage_fp32(mhd_ctx* c, Src<float> s, int what) { stage_launch<float,
 // (a block's kernels are the same however its stencils are asked for)
 void launch_flux_fp32(mhd_ctx* c, Src<float> s) {
     if (c->merged) launch_stage_fp32(c, s, kStageFlux);
-    else flux_launch<float, float, float>(c, s);
+    else flux_launch<float, float, float>(c, s, true);
 }
 
 void launch_emf_fp32(mhd_ctx* c, Src<float> s) {

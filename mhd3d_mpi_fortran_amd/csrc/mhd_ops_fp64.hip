@@ -1,6 +1,7 @@
 // binary64 stencil kernels (compiled with -ffp-contract=off: same operation
 // order as the reference, no fused multiply-add)
 #include "mhd_ops.hpp"
+#include "mhd_sweep.hpp"
 #include "mhd_yee.hpp"
 
 using namespace mhd;
@@ -8,10 +9,12 @@ using namespace mhd;
 void launch_stage_fp64(mhd_ctx* c, Src<double> s, int what) { stage_launch<double, double, double>(c, s, what); }
 
 // (a block's kernels are the same however its stencils are asked for)
-void launch_flux_fp64(mhd_ctx* c, Src<double> s) {
+void launch_flux_fp64(mhd_ctx* c, Src<double> s, bool z) {
     if (c->merged) launch_stage_fp64(c, s, kStageFlux);
-    else flux_launch<double, double, double>(c, s);
+    else flux_launch<double, double, double>(c, s, z);
 }
+
+void launch_sweep_fp64(mhd_ctx* c, Src<double> s, const SweepArgs& a) { sweep_launch(c, s, a); }
 
 void launch_emf_fp64(mhd_ctx* c, Src<double> s) {
     if (c->merged) launch_stage_fp64(c, s, kStageEmf);
