@@ -1184,11 +1184,14 @@ int mhd_flux_stress_old(mhd_ctx* c) { return mhd_flux_stress(c, MHD_STATE_PREDIC
 // reads the extrapolated state written by the predictor
 // The ghost fill rides along; `last`: the CFL partials, which only the next
 // step reads, are wanted
-static void end_of_stage(mhd_ctx* c, bool in_step = false, bool last = true) {
+// `keep`: cell B in binary64 as well, which mixed precision's stages do not read
+// (the stencils take the copies): its Runge-Kutta steps store it with the last
+// stage a call makes, 24 bytes of get_bxyz' 136 a cell before that
+static void end_of_stage(mhd_ctx* c, bool in_step = false, bool last = true, bool keep = true) {
     const bool rk = c->p.stepop != 1;
     // mixed Adams-Bashforth steps take the extrapolated cell B from the faces
     // (k_predict_ab_mixed), so the step itself leaves cell B implicit
-    do_bxyz(c, rk && !mixed(c), rk && mixed(c), last, !(in_step && !rk && mixed(c)), true);
+    do_bxyz(c, rk && !mixed(c), rk && mixed(c), last, !(in_step && mixed(c) && (!rk || !last || !keep)), true);
 }
 // cell B of the current state where a caller reads it
 static void ensure_cellb(mhd_ctx* c) {
@@ -1222,7 +1225,7 @@ int mhd_initialize(mhd_ctx* c, double* tau) {
 
 // step_rk2 / step_rk3 (mhd3d3.f90:3648-3792), in place
 template <int NST>
-static void step_rk(mhd_ctx* c, bool report = false) {
+static void step_rk(mhd_ctx* c, bool report = false, bool keep = true) {
     do_dt(c, false, &c->tau0_host, report);
     double* self[11];
     for (int a = 0; a < 11; ++a) self[a] = *state_slot(c, a);
@@ -1230,7 +1233,7 @@ static void step_rk(mhd_ctx* c, bool report = false) {
         if (st == 1) do_stage<NST, 1>(c, cur_src(c), self);
         else if (st == 2) do_stage<NST, 2>(c, cur_src(c), self);
         else do_stage<NST, 3>(c, cur_src(c), self);
-        end_of_stage(c, true, st == NST);
+        end_of_stage(c, true, st == NST, keep);
     }
 }
 
@@ -1304,8 +1307,8 @@ int mhd_step(mhd_ctx* c, int nsteps, double* tau, double* tau_cfl) {
     for (int n = 0; n < nsteps; ++n) {
         const bool report = n == nsteps - 1;
         if (c->p.stepop == 1) step_ab(c, report);
-        else if (c->p.stepop == 2) step_rk<2>(c, report);
-        else step_rk<3>(c, report);
+        else if (c->p.stepop == 2) step_rk<2>(c, report, report);
+        else step_rk<3>(c, report, report);
     }
     double h[3] = {0., 0., 0.};
     if (nsteps == 0 && hipMemcpyAsync(h, c->scal, 3 * sizeof(double), hipMemcpyDeviceToHost, c->s) != hipSuccess)
