@@ -166,13 +166,14 @@ int mhd_create(mhd_ctx** out, const mhd_params* p) {
     c->ne[2] = (long)(d.nx0 + 1) * (d.ny0 + 1) * d.nz0;
     c->ninterior = (long)d.nx0 * d.ny0 * d.nz0;
     c->emf_fill = kEmfFillThreads;
-    // the two-stream stage pays for its fork and join only on blocks whose
-    // kernels fill the chip for long; small blocks keep one stream
-    c->overlap = c->ninterior >= kOverlapCells;
     if (const char* ev = getenv("MHD_EMF_FILL_THREADS")) c->emf_fill = atol(ev);
     // one launch takes runs of 2 edges, as every EMF of such a block does
     // unless the fill threshold is lowered
-    c->merged = c->ninterior < kOverlapCells && c->emf_fill >= kEmfFillThreads;
+    const long most = p->precision != MHD_MIXED && p->stepop != 1 ? kMergeCellsRK64 : kOverlapCells;
+    c->merged = c->ninterior < most && c->emf_fill >= kEmfFillThreads;
+    // the two-stream stage pays for its fork and join only on blocks whose
+    // kernels fill the chip for long; small blocks keep one stream
+    c->overlap = c->ninterior >= kOverlapCells && !c->merged;
     long nmax = c->ncell;
     nmax = c->nbi > nmax ? c->nbi : nmax;
     nmax = c->nbj > nmax ? c->nbj : nmax;

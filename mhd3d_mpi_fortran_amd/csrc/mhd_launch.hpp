@@ -51,6 +51,13 @@ constexpr long kEmfFillThreads = 256L * 4 * 8 * 64;
 // blocks with at least this many owned cells run a stage on two streams by
 // default (mhd_set_stage_overlap)
 constexpr long kOverlapCells = 1L << 21;
+// binary64 Runge-Kutta blocks keep one launch for a stage's stencils up to this
+// size: PDM RK2 128^3 1376 us a step for 1581 with a launch each on two streams,
+// 176^3 3.73 ms for 4.05, 256^3 11.1 for 11.3; TVD 128^3 1255 for 1296, WENO5 and
+// MPWENO5 equal or 1-2 % less, larger blocks not measured.  (Binary32 EMFs round
+// with their runs' length, so mixed blocks keep theirs; Adams-Bashforth has the
+// z sweep.)
+constexpr long kMergeCellsRK64 = 1L << 25;
 
 // scratch of the binary64 WENO EMF (mhd_emf_weno.hpp): 18 arrays over a
 // slab of whole planes, as many as kWenoScratch bytes hold (it should stay in
