@@ -272,9 +272,11 @@ void *mhd_device_pointer(mhd_ctx *ctx, int which);
  * kernel classes: see MHD_K_*; *ms = summed duration, *launches = count */
 enum { MHD_K_FLUX = 0, MHD_K_EMF = 1, MHD_K_UPDATE = 2, MHD_K_CT = 3, MHD_K_FILL = 4, MHD_K_BXYZ = 5,
        MHD_K_DT = 6, MHD_K_PREV = 7, MHD_K_SURR = 8, MHD_K_NCLASS = 9 };
-/* (blocks below 2^21 owned cells, binary64 Runge-Kutta ones below 2^25, run a stage's PDM or TVD face fluxes and edge
- * EMFs as one launch, which counts as MHD_K_FLUX; there MHD_K_EMF counts EMFs
- * launched by themselves.
+/* (blocks below 2^21 owned cells, binary64 Runge-Kutta ones below 2^25, run a
+ * stage's PDM or TVD face fluxes and edge EMFs as one launch, which counts as
+ * MHD_K_FLUX; there MHD_K_EMF counts EMFs launched by themselves.  Larger
+ * binary64 Adams-Bashforth steps form the z fluxes in the update, which counts
+ * as MHD_K_UPDATE.
  * The learned-reconstruction flux's first pass counts as MHD_K_FLUX;
  * MHD_K_SURR covers its MLP pass over the listed faces, the PDM fallback
  * fix-up, the list reset, sample collection, training and standalone

@@ -921,7 +921,7 @@ static void do_advance_t(mhd_ctx* c, double* const* out) {
 // before the stage ends.  The EMF kernels wait on latency (few waves per
 // SIMD) and CT on HBM, the flux on VALU issue: together they fill the CUs
 // better than one after the other.
-// both: the two in one launch, which blocks below kOverlapCells take (k_stencils)
+// both: the two in one launch, which merged blocks take (k_stencils)
 template <int NST, int ST, typename E, typename F, typename B>
 static void stage_overlapped(mhd_ctx* c, E emf, F flux, B both, double* const* out) {
     auto cells = [&] {

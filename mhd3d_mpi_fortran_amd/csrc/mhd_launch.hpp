@@ -74,7 +74,7 @@ struct mhd_ctx {
     // targets (null = s)
     hipStream_t s2 = nullptr, cur = nullptr;
     hipEvent_t ev_fork = nullptr, ev_emf = nullptr, ev_join = nullptr;
-    bool merged = false;   // one launch for a stage's stencils (blocks below kOverlapCells)
+    bool merged = false;   // one launch for a stage's stencils (kOverlapCells, kMergeCellsRK64)
     bool overlap = true;   // false: one stream, kernels in the reference's order
     bool fused = false;    // mixed Adams-Bashforth PDM steps: fused face flux + update (mhd_set_fusion)
     char* arena = nullptr;
