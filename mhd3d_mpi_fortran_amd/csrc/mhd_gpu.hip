@@ -782,6 +782,12 @@ static void do_fill(mhd_ctx* c) {
     c->dt_fresh = false;
 }
 
+// the grid of every pass that leaves CFL partials over the ghost-inclusive block:
+// one size, whatever else the pass does, as an ensemble's graph reduces the
+// partials of whichever ran last, and workgroups are dealt to the cells by the
+// size of the grid (xcd_block): a part of them is no part of the block
+static dim3 dt_grid(const mhd_ctx* c) { return blocks(c->nbxyz); }
+
 // get_bxyz on the current state, plus (optionally) the ghost fill before it,
 // vf, the fp32 stencil copies and the CFL partials of the next get_dt
 static void do_bxyz(mhd_ctx* c, bool want_vf, bool want_shadow, bool want_dt, bool store_cellb = true,
@@ -795,7 +801,7 @@ static void do_bxyz(mhd_ctx* c, bool want_vf, bool want_shadow, bool want_dt, bo
     const BMet m = bmet(c, want_vf && !mixed(c), want_shadow && mixed(c));
     auto kb = c->met.mode == 2 ? (fill ? k_bxyz<true, true> : k_bxyz<true, false>)
                                : (fill ? k_bxyz<false, true> : k_bxyz<false, false>);
-    const dim3 grid = blocks(fill || sh.rho ? c->nbxyz : c->ncell);
+    const dim3 grid = want_dt ? dt_grid(c) : blocks(fill || sh.rho ? c->nbxyz : c->ncell);
     launch(c, MHD_K_BXYZ, grid, dim3(kBlock), kb, c->d, c->p.gam, c->p.cfl, Faces{c->bi, c->bj, c->bk},
            Cells{c->rho, c->vx, c->vy, c->vz, c->pr}, bc_set(c), store_cellb ? c->bx : (double*)nullptr, c->by, c->bz,
            want_vf ? c->vf : (double*)nullptr, sh, m, sdx(c), sdy(c), sdz(c),
@@ -817,9 +823,9 @@ static void do_dt(mhd_ctx* c, bool set_tau, const double* fixed = nullptr, bool 
     if (!c->dt_fresh && c->cellb_stale) do_bxyz(c, false, false, true);
     long n = c->ndt_valid;
     if (!c->dt_fresh) {
-        launch(c, MHD_K_DT, blocks(c->ncell), dim3(kBlock), k_dt_partial, c->d, c->p.gam, c->p.cfl, cur_state(c),
+        launch(c, MHD_K_DT, dt_grid(c), dim3(kBlock), k_dt_partial, c->d, c->p.gam, c->p.cfl, cur_state(c),
                sdx(c), sdy(c), sdz(c), gmet(c), c->dtpart, c->ncell);
-        n = blocks(c->ncell).x;
+        n = dt_grid(c).x;
     }
     launch(c, MHD_K_DT, dim3(1), dim3(1024), k_dt_final, (const double*)c->dtpart, n, c->scal + SC_DTCFL,
            set_tau || fixed ? c->scal + SC_TAU : (double*)nullptr, fixed ? 1 : 0, fixed ? *fixed : 0.,
@@ -1524,10 +1530,15 @@ int mhd_ensemble_create(mhd_ens** out, mhd_ctx* const* members, int n, const dou
         mhd_ensemble_destroy(e);
         return MHD_ERR_HIP;
     }
-    std::vector<bool> prof(n), ovl(n);
+    // what the host knows of a member's arrays: recording runs nothing
+    struct Known {
+        bool prof, overlap, dt_fresh, cellb_stale;
+        long ndt;
+    };
+    std::vector<Known> known(n);
     for (int a = 0; a < n; ++a) {
-        prof[a] = e->m[a]->prof;
-        ovl[a] = e->m[a]->overlap;
+        const mhd_ctx* c = e->m[a];
+        known[a] = Known{c->prof, c->overlap, c->dt_fresh, c->cellb_stale, c->ndt_valid};
         e->m[a]->prof = false;      // no event records inside the graph
         e->m[a]->overlap = false;   // the members' branches already run side by side
         e->m[a]->tau0_host = tau[a];
@@ -1547,9 +1558,13 @@ int mhd_ensemble_create(mhd_ens** out, mhd_ctx* const* members, int n, const dou
     const bool ended = hipStreamEndCapture(e->root, &g) == hipSuccess;
     e->graph = g;
     for (int a = 0; a < n; ++a) {
-        e->m[a]->prof = prof[a];
-        e->m[a]->overlap = ovl[a];
-        e->m[a]->launch_error = hipSuccess;
+        mhd_ctx* c = e->m[a];
+        c->prof = known[a].prof;
+        c->overlap = known[a].overlap;
+        c->dt_fresh = known[a].dt_fresh;
+        c->cellb_stale = known[a].cellb_stale;
+        c->ndt_valid = known[a].ndt;
+        c->launch_error = hipSuccess;
     }
     ok = ok && ended && g && hipGraphInstantiate(&e->exec, g, nullptr, nullptr, 0) == hipSuccess;
     if (!ok) {
@@ -1566,8 +1581,16 @@ int mhd_ensemble_step(mhd_ens* e, int nsteps) {
     // members' own queued work first, then the graph on the root stream
     for (mhd_ctx* c : e->m)
         if (hipStreamSynchronize(c->s) != hipSuccess) return MHD_ERR_HIP;
-    for (int s = 0; s < nsteps; ++s)
+    for (int s = 0; s < nsteps; ++s) {
         if (hipGraphLaunch(e->exec, e->root) != hipSuccess) return MHD_ERR_HIP;
+        // the last stage's get_bxyz leaves the new state's cell B and partials
+        if (s == 0)
+            for (mhd_ctx* c : e->m) {
+                c->dt_fresh = true;
+                c->ndt_valid = dt_grid(c).x;
+                c->cellb_stale = false;
+            }
+    }
     return hipStreamSynchronize(e->root) == hipSuccess ? MHD_OK : MHD_ERR_HIP;
 }
 
