@@ -272,7 +272,8 @@ void *mhd_device_pointer(mhd_ctx *ctx, int which);
  * kernel classes: see MHD_K_*; *ms = summed duration, *launches = count */
 enum { MHD_K_FLUX = 0, MHD_K_EMF = 1, MHD_K_UPDATE = 2, MHD_K_CT = 3, MHD_K_FILL = 4, MHD_K_BXYZ = 5,
        MHD_K_DT = 6, MHD_K_PREV = 7, MHD_K_SURR = 8, MHD_K_NCLASS = 9 };
-/* (blocks below 2^21 owned cells, binary64 Runge-Kutta ones below 2^25, run a
+/* (blocks below 2^21 owned cells, binary64 Runge-Kutta ones below 2^25 (TVD
+ * 2^22), run a
  * stage's PDM or TVD face fluxes and edge EMFs as one launch, which counts as
  * MHD_K_FLUX; there MHD_K_EMF counts EMFs launched by themselves.  Larger
  * binary64 Adams-Bashforth steps form the z fluxes in the update, which counts
@@ -291,7 +292,7 @@ int mhd_profile_classes(mhd_ctx *ctx, unsigned mask);
 
 /* stage scheduling (no counterpart in the reference): on (the default for
  * blocks of at least 2^21 owned cells, binary64 Runge-Kutta ones of at
- * least 2^25), a stage's edge EMF and CT run on a
+ * least 2^25, 2^22 with TVD), a stage's edge EMF and CT run on a
  * second stream beside its face flux and cell update; off (the default for
  * smaller blocks, and for ensemble members), every kernel runs on the
  * context's stream in the reference's order (the per-kernel times then add

@@ -167,10 +167,9 @@ int mhd_create(mhd_ctx** out, const mhd_params* p) {
     c->ninterior = (long)d.nx0 * d.ny0 * d.nz0;
     c->emf_fill = kEmfFillThreads;
     if (const char* ev = getenv("MHD_EMF_FILL_THREADS")) c->emf_fill = atol(ev);
-    // one launch takes runs of 2 edges, as every EMF of such a block does
-    // unless the fill threshold is lowered
-    const long most = p->precision != MHD_MIXED && p->stepop != 1 ? kMergeCellsRK64 : kOverlapCells;
-    c->merged = c->ninterior < most && c->emf_fill >= kEmfFillThreads;
+    // the one launch takes short runs of edges (stage_launch_mm), so a lowered
+    // fill threshold, which asks for long ones, keeps it off
+    c->merged = c->ninterior < merge_cells(*p) && c->emf_fill >= kEmfFillThreads;
     // the two-stream stage pays for its fork and join only on blocks whose
     // kernels fill the chip for long; small blocks keep one stream
     c->overlap = c->ninterior >= kOverlapCells && !c->merged;

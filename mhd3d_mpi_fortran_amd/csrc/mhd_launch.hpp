@@ -49,15 +49,29 @@ struct SurrogateState;
 // short runs
 constexpr long kEmfFillThreads = 256L * 4 * 8 * 64;
 // blocks with at least this many owned cells run a stage on two streams by
-// default (mhd_set_stage_overlap)
+// default (mhd_set_stage_overlap), smaller ones its stencils in one launch
+// (k_stencils)
 constexpr long kOverlapCells = 1L << 21;
-// binary64 Runge-Kutta blocks keep one launch for a stage's stencils up to this
-// size: PDM RK2 128^3 1376 us a step for 1581 with a launch each on two streams,
-// 176^3 3.73 ms for 4.05, 256^3 11.1 for 11.3; TVD 128^3 1255 for 1296, WENO5 and
-// MPWENO5 equal or 1-2 % less, larger blocks not measured.  (Binary32 EMFs round
-// with their runs' length, so mixed blocks keep theirs; Adams-Bashforth has the
-// z sweep.)
-constexpr long kMergeCellsRK64 = 1L << 25;
+// Binary64 Runge-Kutta blocks keep the one launch up to the size to which it is the
+// faster one by measurement (a launch each on two streams in brackets):
+//   PDM   128^3 1393 us a step (1585), 160^3 2889 (3183), 200^3 5875 (6343), 256^3
+//         11.23 ms (11.35), 300^3 18.52 (18.57), 320^3 21.78 (21.84)
+//   TVD   128^3 1265 us (1299), 144^3 1961 (1997), 160^3 2588 (2591), 200^3 5183
+//         (5186), 300^3 16.87 ms (16.63): from 200^3 on the launches of their own
+//         take runs of 16 edges, the one launch runs of 2
+//   WENO5 and MPWENO5 (whose EMF has launches of its own either way) 128^3 3240 and
+//         4522 us (3235, 4555), 200^3 12.98 and 18.16 ms (12.96, 18.17), 256^3 26.03
+//         and 36.57 (26.13, 36.69), 300^3 43.32 and 58.90 (43.88, 58.96); long thin
+//         blocks of 3 M cells within 1 % either way
+// Eight cells along x: PDM 8 x 600 x 600 6.74 ms (8.14), 8 x 1800 x 1800 62.4 (64.8);
+// TVD 8 x 600 x 600 5.72 (5.62).  (Binary32 EMFs round with their runs' length, so
+// mixed blocks keep theirs; Adams-Bashforth has the z sweep.)
+constexpr long kMergeCells64 = 1L << 25, kMergeCellsTvd64 = 1L << 22;
+// the bound for a block of these parameters
+inline long merge_cells(const mhd_params& p) {
+    if (p.precision == MHD_MIXED || p.stepop == 1) return kOverlapCells;
+    return p.reconop == mhd::TVD ? kMergeCellsTvd64 : kMergeCells64;
+}
 
 // scratch of the binary64 WENO EMF (mhd_emf_weno.hpp): 18 arrays over a
 // slab of whole planes, as many as kWenoScratch bytes hold (it should stay in
@@ -74,7 +88,7 @@ struct mhd_ctx {
     // targets (null = s)
     hipStream_t s2 = nullptr, cur = nullptr;
     hipEvent_t ev_fork = nullptr, ev_emf = nullptr, ev_join = nullptr;
-    bool merged = false;   // one launch for a stage's stencils (kOverlapCells, kMergeCellsRK64)
+    bool merged = false;   // one launch for a stage's stencils (merge_cells)
     bool overlap = true;   // false: one stream, kernels in the reference's order
     bool fused = false;    // mixed Adams-Bashforth PDM steps: fused face flux + update (mhd_set_fusion)
     char* arena = nullptr;
