@@ -277,7 +277,8 @@ enum { MHD_K_FLUX = 0, MHD_K_EMF = 1, MHD_K_UPDATE = 2, MHD_K_CT = 3, MHD_K_FILL
  * stage's PDM or TVD face fluxes and edge EMFs as one launch, which counts as
  * MHD_K_FLUX; there MHD_K_EMF counts EMFs launched by themselves.  Larger
  * binary64 Adams-Bashforth steps form the z fluxes in the update, which counts
- * as MHD_K_UPDATE.
+ * as MHD_K_UPDATE, unless the block is narrow along x (PDM then takes the one
+ * launch).
  * The learned-reconstruction flux's first pass counts as MHD_K_FLUX;
  * MHD_K_SURR covers its MLP pass over the listed faces, the PDM fallback
  * fix-up, the list reset, sample collection, training and standalone

@@ -835,7 +835,7 @@ static void do_dt(mhd_ctx* c, bool set_tau, const double* fixed = nullptr, bool 
 // (mhd_sweep.hpp); Runge-Kutta updates in place the cells whose neighbours'
 // fluxes are still to be formed
 static bool can_sweep(const mhd_ctx* c) {
-    return !mixed(c) && c->p.stepop == 1 && !c->merged && !c->p.surrogate && c->met.mode != 2;
+    return !mixed(c) && c->p.stepop == 1 && !c->merged && !c->p.surrogate && c->met.mode != 2 && sweep_fills(c->p);
 }
 static SweepArgs sweep_args(const mhd_ctx* c, double* const* out, bool keep) {
     SweepArgs a{};

@@ -65,11 +65,28 @@ constexpr long kOverlapCells = 1L << 21;
 //         blocks of 3 M cells within 1 % either way
 // Eight cells along x: PDM 8 x 600 x 600 6.74 ms (8.14), 8 x 1800 x 1800 62.4 (64.8);
 // TVD 8 x 600 x 600 5.72 (5.62).  (Binary32 EMFs round with their runs' length, so
-// mixed blocks keep theirs; Adams-Bashforth has the z sweep.)
+// mixed blocks keep theirs.)
 constexpr long kMergeCells64 = 1L << 25, kMergeCellsTvd64 = 1L << 22;
-// the bound for a block of these parameters
+// Whether the rows of a binary64 Adams-Bashforth block fill enough of the sweep's
+// 64-lane tiles (mhd_sweep.hpp; lanes past a row's end form a flux and drop it).
+// Flux and update of their own in brackets.  PDM from 1/2 on: 33 x 260 x 260 1264 us
+// (1268; a narrower one takes the one launch, merge_cells: 24 x 320 x 320 1454 for the
+// sweep's 1654); TVD from 3/8 on: 24 x 320 x 320 1264 us (1280), 20 x 400 x 400 1795
+// (1797), 16 x 400 x 400 1697 (1679), 8 x 400 x 800 2835 (2726); WENO5 and MPWENO5 from
+// 3/4 on: 100 x 160 x 160 2145 and 2984 us (2171, 3022), 48 x 220 x 220 2046 and 2856
+// (2046, 2842), 65 x 190 x 190 2349 and 3291 (2246, 3184).
+inline bool sweep_fills(const mhd_params& p) {
+    const int lanes = (p.nx0 + mhd::kTileX - 1) / mhd::kTileX * mhd::kTileX;
+    const int eighths = p.reconop == mhd::PDM ? 4 : (p.reconop == mhd::TVD ? 3 : 6);
+    return 8 * p.nx0 >= eighths * lanes;
+}
+// the bound for a block of these parameters.  Adams-Bashforth blocks past it have the
+// sweep; PDM ones too narrow for that keep the one launch: 16 x 400 x 400 1941 us
+// (sweep 2285, a launch each 2269), 8 x 400 x 800 3213 (3961, 3842), 16 x 1400 x 1400
+// 24.5 ms (25.2, 25.5)
 inline long merge_cells(const mhd_params& p) {
-    if (p.precision == MHD_MIXED || p.stepop == 1) return kOverlapCells;
+    if (p.precision == MHD_MIXED) return kOverlapCells;
+    if (p.stepop == 1) return p.reconop == mhd::PDM && !sweep_fills(p) ? kMergeCells64 : kOverlapCells;
     return p.reconop == mhd::TVD ? kMergeCellsTvd64 : kMergeCells64;
 }
 
