@@ -49,7 +49,9 @@ typedef struct {
     int reconop;         /* 1 PDM, 2 TVD (van Leer), 3 WENO5, 4 MPWENO5 */
     int stepop;          /* 1 Adams-Bashforth, 2 TVD RK2, 3 TVD RK3 */
     int bc[3];           /* per axis: MHD_BC_EVEN (reference) or MHD_BC_PERIODIC */
-    int precision;       /* MHD_FP64, or MHD_MIXED: fp32 stencils/fluxes/EMF,
+    int precision;       /* MHD_FP64 (the reference's operations; numerators below
+                            1e-289 may be divided to one place of the last), or
+                            MHD_MIXED: fp32 stencils/fluxes/EMF,
                             fp64 conserved accumulation and CT update */
     int surrogate;       /* 0, or 1: learned face reconstruction for the flux
                             (needs mhd_surrogate_set_weights), PDM fallback */

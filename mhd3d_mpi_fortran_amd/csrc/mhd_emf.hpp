@@ -27,6 +27,8 @@ struct VavFoot<TVD> {
     static constexpr int N = 4, LO = -2;
 };
 template <>
+struct VavFoot<TVD_FULL> : VavFoot<TVD> {};
+template <>
 struct VavFoot<WENO5> {
     static constexpr int N = 6, LO = -3;
 };
@@ -95,10 +97,11 @@ struct VavWin {
 template <typename R, int M, bool MD1, bool U>
 __device__ __forceinline__ R vav_win(const VavWin<R, M, MD1, U>& W, const Coef<R>& c, const R* g = nullptr) {
     R v00_0, v10_0, v01_0, v11_0, v00_1, v01_1, v10_1, v11_1;
-    if constexpr (M == TVD) {
+    if constexpr (scheme(M) == TVD) {
         const R vi = (W.cv(-1, -1) + W.cv(0, -1) + W.cv(0, 0) + W.cv(-1, 0)) / R(4);
-        tvd(W.cv(-2, 0), W.cv(-1, 0), W.cv(0, 0), W.cv(1, 0), vi, c.eps, v00_0, v10_0);
-        tvd(W.cv(0, -2), W.cv(0, -1), W.cv(0, 0), W.cv(0, 1), vi, c.eps, v00_1, v01_1);
+        constexpr bool FULL = M == TVD_FULL;
+        tvd<R, FULL>(W.cv(-2, 0), W.cv(-1, 0), W.cv(0, 0), W.cv(1, 0), vi, c.eps, v00_0, v10_0);
+        tvd<R, FULL>(W.cv(0, -2), W.cv(0, -1), W.cv(0, 0), W.cv(0, 1), vi, c.eps, v00_1, v01_1);
         v10_1 = v00_1;
         v11_1 = v01_1;
         v01_0 = v00_0;

@@ -169,7 +169,8 @@ int mhd_create(mhd_ctx** out, const mhd_params* p) {
     if (const char* ev = getenv("MHD_EMF_FILL_THREADS")) c->emf_fill = atol(ev);
     // the one launch takes short runs of edges (stage_launch_mm), so a lowered
     // fill threshold, which asks for long ones, keeps it off
-    c->merged = c->ninterior < merge_cells(*p) && c->emf_fill >= kEmfFillThreads;
+    c->merged = c->ninterior < merge_cells(*p) && c->emf_fill >= kEmfFillThreads &&
+                (p->precision == MHD_MIXED || !full_division(*p));
     // the two-stream stage pays for its fork and join only on blocks whose
     // kernels fill the chip for long; small blocks keep one stream
     c->overlap = c->ninterior >= kOverlapCells && !c->merged;
@@ -296,6 +297,9 @@ void mhd_destroy(mhd_ctx* c) {
 }
 
 static int upload_metric_spacing(mhd_ctx* c);
+static bool mid_range(const std::vector<double>& h) {
+    return std::all_of(h.begin(), h.end(), [](double x) { return x >= 0x1p-400 && x <= 0x1p400; });
+}
 static void ensure_cellb(mhd_ctx* c);
 
 int mhd_set_geometry(mhd_ctx* c, const double* dx, const double* dy, const double* dz) {
@@ -322,6 +326,7 @@ int mhd_set_geometry(mhd_ctx* c, const double* dx, const double* dy, const doubl
             if (!(h[g - 1] == h[g + n0[a] - 1]) || !(h[hi - 1] == h[hi - n0[a] - 1])) c->ghost_twins = false;
         }
     }
+    c->spacing_mid = mid_range(c->hdx) && mid_range(c->hdy) && mid_range(c->hdz);
     if (c->met.on && upload_metric_spacing(c) != MHD_OK) return MHD_ERR_HIP;
     return hipStreamSynchronize(c->s) == hipSuccess ? MHD_OK : MHD_ERR_HIP;
 }
@@ -334,9 +339,11 @@ static int upload_metric_spacing(mhd_ctx* c) {
     std::vector<double> h;
     const std::vector<double>* src[3] = {&c->hdx, &c->hdy, &c->hdz};
     double* dst[3] = {c->dxm, c->dym, c->dzm};
+    c->spacing_mid = true;
     for (int a = 0; a < 3; ++a) {
         h.resize(src[a]->size());
         for (size_t q = 0; q < h.size(); ++q) h[q] = (*src[a])[q] / c->met.g[a];
+        c->spacing_mid = c->spacing_mid && mid_range(h);
         if (hipMemcpy(dst[a], h.data(), h.size() * sizeof(double), hipMemcpyHostToDevice) != hipSuccess)
             return MHD_ERR_HIP;
     }
@@ -832,10 +839,12 @@ static void do_dt(mhd_ctx* c, bool set_tau, const double* fixed = nullptr, bool 
 }
 
 // a binary64 Adams-Bashforth stage's z fluxes and update in one kernel
-// (mhd_sweep.hpp); Runge-Kutta updates in place the cells whose neighbours'
+// (mhd_sweep.hpp), whose divisions by the spacings and by the limiters'
+// differences have Divisor's range; Runge-Kutta updates in place the cells whose neighbours'
 // fluxes are still to be formed
 static bool can_sweep(const mhd_ctx* c) {
-    return !mixed(c) && c->p.stepop == 1 && !c->merged && !c->p.surrogate && c->met.mode != 2 && sweep_fills(c->p);
+    return !mixed(c) && c->p.stepop == 1 && !c->merged && !c->p.surrogate && c->met.mode != 2 && sweep_fills(c->p) &&
+           c->spacing_mid && !full_division(c->p);
 }
 static SweepArgs sweep_args(const mhd_ctx* c, double* const* out, bool keep) {
     SweepArgs a{};

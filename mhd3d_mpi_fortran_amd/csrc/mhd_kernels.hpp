@@ -165,7 +165,7 @@ __device__ __forceinline__ void face_flux_vals(const Coef<R>& c, const R* l, con
     R v0, v1;
     // left state, positive half-moments
     const R unl = D == 1 ? ul : (D == 2 ? vl : wl);
-    R leng = R(.5) * rl * (sq(ul) + sq(vl) + sq(wl)) + qdiv(pl, c.gm1);
+    R leng = R(.5) * rl * (sq(ul) + sq(vl) + sq(wl)) + ldiv<R, false>(pl, c.gm1);
     R lam = qdiv(rl, R(2) * pl);
     vface<R>(lam, unl, +1, c.rspi, v0, v1);
     R fr0 = rl * v1, fmx = rl * ul * v1, fmy = rl * vl * v1, fmz = rl * wl * v1;
@@ -184,7 +184,7 @@ __device__ __forceinline__ void face_flux_vals(const Coef<R>& c, const R* l, con
 
     // right state, negative half-moments
     const R unr = D == 1 ? ur : (D == 2 ? vr : wr);
-    leng = R(.5) * rr * (sq(ur) + sq(vr) + sq(wr)) + qdiv(pr, c.gm1);
+    leng = R(.5) * rr * (sq(ur) + sq(vr) + sq(wr)) + ldiv<R, false>(pr, c.gm1);
     lam = qdiv(rr, R(2) * pr);
     vface<R>(lam, unr, -1, c.rspi, v0, v1);
     R gr0 = rr * v1, gmx = rr * ur * v1, gmy = rr * vr * v1, gmz = rr * wr * v1;
@@ -256,7 +256,7 @@ __device__ __forceinline__ void face_flux_met_vals(const Coef<R>& c, const R* l,
     {
         const R rl = l[0], ul = l[1], vl = l[2], wl = l[3], pl = l[4], bxl = l[5], byl = l[6], bzl = l[7];
         const R un = n[0] * ul + n[1] * vl + n[2] * wl;
-        const R leng = R(.5) * rl * (sq(ul) + sq(vl) + sq(wl)) + qdiv(pl, c.gm1);
+        const R leng = R(.5) * rl * (sq(ul) + sq(vl) + sq(wl)) + ldiv<R, false>(pl, c.gm1);
         R lam = qdiv(rl, R(2) * pl);
         vface<R>(lam, un, +1, c.rspi, v0, v1);
         fx[0] = rl * v1;
@@ -276,7 +276,7 @@ __device__ __forceinline__ void face_flux_met_vals(const Coef<R>& c, const R* l,
     {
         const R rr = r[0], ur = r[1], vr = r[2], wr = r[3], pr = r[4], bxr = r[5], byr = r[6], bzr = r[7];
         const R un = n[0] * ur + n[1] * vr + n[2] * wr;
-        const R leng = R(.5) * rr * (sq(ur) + sq(vr) + sq(wr)) + qdiv(pr, c.gm1);
+        const R leng = R(.5) * rr * (sq(ur) + sq(vr) + sq(wr)) + ldiv<R, false>(pr, c.gm1);
         R lam = qdiv(rr, R(2) * pr);
         vface<R>(lam, un, -1, c.rspi, v0, v1);
         fx[0] += rr * v1;

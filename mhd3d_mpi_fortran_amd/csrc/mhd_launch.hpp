@@ -135,6 +135,7 @@ struct mhd_ctx {
     float* sh[12] = {};
     bool dt_fresh = false;   // dtpart holds the CFL partials of the current state
     long ndt_valid = 0;      // ... that many of them
+    bool spacing_mid = false;  // the update's spacings lie within 2^-400 .. 2^400
     bool ghost_twins = false;  // every ghost cell repeats an owned cell (periodic axes, equal ghost spacings)
     bool cellb_stale = false;  // bx,by,bz not stored for the current state (mixed AB steps, uploads, advances)
     bool pred_valid = false;   // the extrapolated state of mhd_predict_ab is held (xh / fp32 copies)
@@ -216,6 +217,12 @@ inline void launch(mhd_ctx* c, int kclass, dim3 g, dim3 b, void (*k)(KArgs...), 
     }
 }
 
+// the binary64 reconstruction of a context (mhd::Recon)
+inline bool full_division(const mhd_params& p) {  // needed by the limiters, for its eps
+    return p.reconop != mhd::PDM && mhd::Coef<double>::full(p.eps);
+}
+inline int recon_code(const mhd_ctx* c) { return full_division(c->p) ? c->p.reconop + 3 : c->p.reconop; }
+
 template <typename R>
 inline mhd::Coef<R> make_coef(const mhd_ctx* c) {
     mhd::Coef<R> k;
@@ -228,6 +235,7 @@ inline mhd::Coef<R> make_coef(const mhd_ctx* c) {
     k.alpha = R(c->p.alpha);
     k.beta = R(c->p.beta);
     k.rspi = R(std::sqrt(pi));
+    if constexpr (sizeof(R) == 8) k.set_weno();
     return k;
 }
 

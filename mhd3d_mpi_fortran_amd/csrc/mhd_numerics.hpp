@@ -8,18 +8,42 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+#include <cmath>
 #include <cstddef>
 #include <cstdint>
 
 namespace mhd {
 
-enum Recon { PDM = 1, TVD = 2, WENO5 = 3, MPWENO5 = 4 };
+// The limiters of the last three divide by differences plus eps; for eps too small to
+// keep such a divisor within Divisor's range (Coef<double>::full) binary64 takes
+// them with the compiler's division
+enum Recon { PDM = 1, TVD = 2, WENO5 = 3, MPWENO5 = 4, TVD_FULL = 5, WENO5_FULL = 6, MPWENO5_FULL = 7 };
+constexpr int scheme(int m) { return m > MPWENO5 ? m - 3 : m; }
 
 // scalar parameters of the scheme (module pars, mhd3d3.f90:87-91)
 template <typename R>
 struct Coef {
     R gam, gm1, cfl, pdmb, eps, alpha, beta;
     R rspi;  // sqrt(pi) of the binary64 pi = 4*atan(1) (mhd3d3.f90:39), host libm
+};
+template <>
+struct Coef<double> {
+    double gam, gm1, cfl, pdmb, eps, alpha, beta;
+    double rspi;
+    // numerators of the WENO weights .1, .6, .3 times a power of two, which the
+    // weights' normalisation takes out again: without it the three quotients and
+    // their sum are subnormal, and lose bits, for fields of 1e76 and more.  With
+    // eps >= 2^-400 the divisors (eps + s)^2 are at least 2^-800; the power keeps
+    // the quotients between 2^-830 and 2^1000.
+    double wn[3];
+    static bool full(double eps) { return !(eps >= 0x1p-400); }
+    void set_weno() {
+        const double m = full(eps) ? 1. : std::ldexp(1., std::min(900, 1000 + 2 * std::ilogb(eps)));
+        wn[0] = .1 * m;
+        wn[1] = .6 * m;
+        wn[2] = .3 * m;
+    }
 };
 
 template <typename R>
@@ -29,18 +53,24 @@ __device__ __forceinline__ R sq(R x) { return x * x; }
 // reference's arithmetic); in fp32 (mixed precision) the hardware
 // reciprocal and square root (1 ulp), which skip the range-scaling
 // sequence of the correctly rounded forms
-//
-// Binary64 divides by Newton's iteration on the hardware reciprocal: two
-// steps give 1/b to its last place, the quotient a * (1/b) is corrected by
-// its exact remainder (fused multiply-add), and v_div_fixup supplies the
-// infinities, zeros, NaNs and signs.  That is the compiler's own division
-// without its two range-scaling instructions and the VCC chain between them
-// (9 VALU instructions instead of 11), so it rounds like it wherever the
-// remainder is representable: |a| above 2^-960 and |b|, |a/b| within
-// 2^+-1000, far beyond any quantity the stencils divide.  The
-// WENO weights' three quotients share one reciprocal (17 instructions for 33).
-// At 96 x 64 x 128 (WENO5) the y flux takes 107 us for 124, the EMF 363 for
-// 443; at 256^3 (PDM) the step 6.57 ms for 6.81.
+template <typename R>
+__device__ __forceinline__ R qdiv(R a, R b) { return a / b; }
+template <>
+__device__ __forceinline__ float qdiv<float>(float a, float b) { return a * __builtin_amdgcn_rcpf(b); }
+
+// Division by Newton's iteration on the hardware reciprocal, for divisors of 2^-1024
+// and more: two steps give 1/b to its last place, the quotient a * (1/b) is
+// corrected by its exact remainder (fused multiply-add), and v_div_fixup supplies
+// the infinities, zeros, NaNs and signs.  That is the compiler's own division
+// without its two range-scaling instructions and the VCC chain between them (9 VALU
+// instructions instead of 11), so it rounds like it wherever the remainder is
+// representable (|a| above 2^-960; below, the quotient may be one place off).  A
+// smaller divisor gives infinity where a quotient may exist: the limiters' are
+// kept from that by eps (Coef<double>), and gam - 1 is 0 or at least 2^-53.  The
+// flux divides by a pressure as well, which nothing bounds, and has the compiler's
+// division there (256^3 PDM step 5.91 ms, 6.04 with this one; 64^3 TVD 874 us, 864).  The WENO weights' three quotients share one reciprocal (17
+// instructions for 33).  At 96 x 64 x 128 (WENO5) the y flux takes 107 us for 124,
+// the EMF 363 for 443.
 template <typename R>
 struct Divisor {
     R b, y;  // y = 1/b
@@ -60,8 +90,8 @@ struct Divisor<float> {
     __device__ __forceinline__ explicit Divisor(float d) : y(__builtin_amdgcn_rcpf(d)) {}
     __device__ __forceinline__ float under(float a) const { return a * y; }
 };
-template <typename R>
-__device__ __forceinline__ R qdiv(R a, R b) { return Divisor<R>(b).under(a); }
+template <typename R, bool FULL>
+__device__ __forceinline__ R ldiv(R a, R b) { return FULL ? a / b : Divisor<R>(b).under(a); }
 template <typename R>
 __device__ __forceinline__ R qsqrt(R x) { return sqrt(x); }
 // division by a constant of few significant bits (840, 6, 3): the rounded
@@ -69,7 +99,8 @@ __device__ __forceinline__ R qsqrt(R x) { return sqrt(x); }
 // exact remainder: the corrected value is within 2^-52 of an ulp of x/c, and
 // x/c lies at least 2^-8 of an ulp from any midpoint between two doubles
 // (their distance is a multiple of ulp/2 over c's odd part), so it rounds
-// like x / c.  fp32 multiplies by the rounded reciprocal.
+// like x / c (|x| above 2^-960; below it may be a unit of the subnormal numbers
+// off).  fp32 multiplies by the rounded reciprocal.
 template <typename R>
 __device__ __forceinline__ R cdiv(R x, double c) {
     const R y = R(1. / c), q = x * y;
@@ -127,13 +158,13 @@ __device__ __forceinline__ void pdm2(R fm2, R fm1, R f0, R fp1, R fi, R pdmb, R&
 }
 
 // TVD van Leer (mhd3d3.f90:1240-1246)
-template <typename R>
+template <typename R, bool FULL = false>
 __device__ __forceinline__ void tvd(R fm2, R fm1, R f0, R fp1, R fi, R eps, R& fl, R& fr) {
-    R a = qdiv(fm1 - fm2, f0 - fm1 + eps);
-    R b = qdiv(a + fabs(a), R(1) + fabs(a));
+    R a = ldiv<R, FULL>(fm1 - fm2, f0 - fm1 + eps);
+    R b = ldiv<R, FULL>(a + fabs(a), R(1) + fabs(a));
     fl = fm1 - b * (fm1 - fi);
-    a = qdiv(f0 - fp1, fm1 - f0 + eps);
-    b = qdiv(a + fabs(a), R(1) + fabs(a));
+    a = ldiv<R, FULL>(f0 - fp1, fm1 - f0 + eps);
+    b = ldiv<R, FULL>(a + fabs(a), R(1) + fabs(a));
     fr = f0 - b * (f0 - fi);
 }
 
@@ -146,27 +177,51 @@ __device__ __forceinline__ float tvd_b(float n, float d) {
     return (n != 0.f && ((n > 0.f) == (d >= 0.f))) ? 2.f * n * __builtin_amdgcn_rcpf(n + d) : 0.f;
 }
 template <>
-__device__ __forceinline__ void tvd<float>(float fm2, float fm1, float f0, float fp1, float fi, float eps, float& fl,
+__device__ __forceinline__ void tvd<float, false>(float fm2, float fm1, float f0, float fp1, float fi, float eps, float& fl,
                                            float& fr) {
     fl = fm1 - tvd_b(fm1 - fm2, f0 - fm1 + eps) * (fm1 - fi);
     fr = f0 - tvd_b(f0 - fp1, fm1 - f0 + eps) * (f0 - fi);
 }
 
+// weights of one WENO5 side from the smoothness indicators s
+template <typename R, bool FULL>
+__device__ __forceinline__ void weno_weights(R s0, R s1, R s2, const Coef<R>& c, R& w0, R& w1, R& w2) {
+    const R eps = c.eps;
+    if constexpr (FULL) {
+        s0 = R(.1) / sq(eps + s0);
+        s1 = R(.6) / sq(eps + s1);
+        s2 = R(.3) / sq(eps + s2);
+        const R t = s0 + s1 + s2;
+        w0 = s0 / t;
+        w1 = s1 / t;
+        w2 = s2 / t;
+    } else {
+        R n0 = R(.1), n1 = R(.6), n2 = R(.3);
+        if constexpr (sizeof(R) == 8) {
+            n0 = c.wn[0];
+            n1 = c.wn[1];
+            n2 = c.wn[2];
+        }
+        s0 = ldiv<R, false>(n0, sq(eps + s0));
+        s1 = ldiv<R, false>(n1, sq(eps + s1));
+        s2 = ldiv<R, false>(n2, sq(eps + s2));
+        R t = s0 + s1 + s2;
+        const Divisor<R> dt(t);   // one reciprocal serves the three weights
+        w0 = dt.under(s0), w1 = dt.under(s1), w2 = dt.under(s2);
+    }
+}
+
 // one side of WENO5 (mhd3d3.f90:1335-1356); mirrored arguments give the right side
-template <typename R>
-__device__ __forceinline__ R weno5_side(R fm3, R fm2, R fm1, R f0, R fp1, R eps) {
+template <typename R, bool FULL>
+__device__ __forceinline__ R weno5_side(R fm3, R fm2, R fm1, R f0, R fp1, const Coef<R>& c) {
     R h0 = cdiv<R>(R(2) * fm3 - R(7) * fm2 + R(11) * fm1, 6.);
     R h1 = cdiv<R>(-fm2 + R(5) * fm1 + R(2) * f0, 6.);
     R h2 = cdiv<R>(R(2) * fm1 + R(5) * f0 - fp1, 6.);
     R s0 = R(13. / 12.) * sq(fm3 - R(2) * fm2 + fm1) + R(.25) * sq(fm3 - R(4) * fm2 + R(3) * fm1);
     R s1 = R(13. / 12.) * sq(fm2 - R(2) * fm1 + f0) + R(.25) * sq(fm2 - f0);
     R s2 = R(13. / 12.) * sq(fm1 - R(2) * f0 + fp1) + R(.25) * sq(R(3) * fm1 - R(4) * f0 + fp1);
-    s0 = qdiv(R(.1), sq(eps + s0));
-    s1 = qdiv(R(.6), sq(eps + s1));
-    s2 = qdiv(R(.3), sq(eps + s2));
-    R t = s0 + s1 + s2;
-    const Divisor<R> dt(t);   // one reciprocal serves the three weights
-    R w0 = dt.under(s0), w1 = dt.under(s1), w2 = dt.under(s2);
+    R w0, w1, w2;
+    weno_weights<R, FULL>(s0, s1, s2, c, w0, w1, w2);
     return w0 * h0 + w1 * h1 + w2 * h2;
 }
 
@@ -220,32 +275,44 @@ struct Stencil<R, PDM> {
         pdm2(s[2], s[3], s[4], s[5], fi, c.pdmb, fl, fr);
     }
 };
-template <typename R>
-struct Stencil<R, TVD> {
+template <typename R, bool FULL>
+struct StencilTvd {
     static constexpr int lo = -2, n = 4;
     __device__ static __forceinline__ void run(const R* s, const Coef<R>& c, R& fl, R& fr) {
         R fi = (s[1] + s[2]) / R(2);
-        tvd(s[0], s[1], s[2], s[3], fi, c.eps, fl, fr);
+        tvd<R, FULL>(s[0], s[1], s[2], s[3], fi, c.eps, fl, fr);
     }
 };
-template <typename R>
-struct Stencil<R, WENO5> {
+template <typename R, bool FULL>
+struct StencilWeno5 {
     static constexpr int lo = -3, n = 6;
     __device__ static __forceinline__ void run(const R* s, const Coef<R>& c, R& fl, R& fr) {
-        fl = weno5_side(s[0], s[1], s[2], s[3], s[4], c.eps);
-        fr = weno5_side(s[5], s[4], s[3], s[2], s[1], c.eps);
+        fl = weno5_side<R, FULL>(s[0], s[1], s[2], s[3], s[4], c);
+        fr = weno5_side<R, FULL>(s[5], s[4], s[3], s[2], s[1], c);
     }
 };
-template <typename R>
-struct Stencil<R, MPWENO5> {
+template <typename R, bool FULL>
+struct StencilMpweno5 {
     static constexpr int lo = -3, n = 6;
     __device__ static __forceinline__ void run(const R* s, const Coef<R>& c, R& fl, R& fr) {
-        R wl = weno5_side(s[0], s[1], s[2], s[3], s[4], c.eps);
-        R wr = weno5_side(s[5], s[4], s[3], s[2], s[1], c.eps);
+        R wl = weno5_side<R, FULL>(s[0], s[1], s[2], s[3], s[4], c);
+        R wr = weno5_side<R, FULL>(s[5], s[4], s[3], s[2], s[1], c);
         fl = mp_side(wl, s[0], s[1], s[2], s[3], s[4], c.alpha, c.beta);
         fr = mp_side(wr, s[5], s[4], s[3], s[2], s[1], c.alpha, c.beta);
     }
 };
+template <typename R>
+struct Stencil<R, TVD> : StencilTvd<R, false> {};
+template <typename R>
+struct Stencil<R, WENO5> : StencilWeno5<R, false> {};
+template <typename R>
+struct Stencil<R, MPWENO5> : StencilMpweno5<R, false> {};
+template <typename R>
+struct Stencil<R, TVD_FULL> : StencilTvd<R, true> {};
+template <typename R>
+struct Stencil<R, WENO5_FULL> : StencilWeno5<R, true> {};
+template <typename R>
+struct Stencil<R, MPWENO5_FULL> : StencilMpweno5<R, true> {};
 
 // reconstruct the face between cells base-stride and base of array f
 template <typename R, int M, typename T>

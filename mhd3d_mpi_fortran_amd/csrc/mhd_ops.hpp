@@ -21,7 +21,7 @@ namespace mhd {
 // 0.72 vs 0.53 ms).
 template <int M, int K>
 struct EmfSteps {
-    static constexpr int T = (M == TVD || (M == PDM && K == 1)) ? 16 : 8;
+    static constexpr int T = (scheme(M) == TVD || (M == PDM && K == 1)) ? 16 : 8;
     static constexpr int T_SHORT = 2;
 };
 
@@ -111,6 +111,13 @@ void flux_launch_m(mhd_ctx* c, Src<TI> s, bool z) {
 
 template <typename R, typename TI, typename TF>
 void flux_launch(mhd_ctx* c, Src<TI> s, bool z) {
+    if constexpr (sizeof(R) == 8) {
+        switch (recon_code(c)) {
+        case TVD_FULL: flux_launch_m<R, TI, TF, TVD_FULL>(c, s, z); return;
+        case WENO5_FULL: flux_launch_m<R, TI, TF, WENO5_FULL>(c, s, z); return;
+        case MPWENO5_FULL: flux_launch_m<R, TI, TF, MPWENO5_FULL>(c, s, z); return;
+        }
+    }
     switch (c->p.reconop) {
     case PDM: flux_launch_m<R, TI, TF, PDM>(c, s, z); break;
     case TVD: flux_launch_m<R, TI, TF, TVD>(c, s, z); break;
@@ -199,7 +206,7 @@ void emf_launch_m(mhd_ctx* c, Src<TI> s) {
     // edges they serve; in fp32 the march stays: which products of a line its
     // compiler contracts depends on the line's place in the footprint, so
     // shared lines would round differently by up to 2e-7 of an edge's EMF
-    if constexpr ((M == WENO5 || M == MPWENO5) && sizeof(R) == 8) {
+    if constexpr ((scheme(M) == WENO5 || scheme(M) == MPWENO5) && sizeof(R) == 8) {
         emf_weno_launch<R, M, TI, TF>(c, u, s);
     } else {
         emf_launch_k<R, M, 1, TI, TF>(c, EmfIn<TI>{u[1], u[2], s.bj, s.bk, s.vf});
@@ -210,6 +217,13 @@ void emf_launch_m(mhd_ctx* c, Src<TI> s) {
 
 template <typename R, typename TI, typename TF>
 void emf_launch(mhd_ctx* c, Src<TI> s) {
+    if constexpr (sizeof(R) == 8) {
+        switch (recon_code(c)) {
+        case TVD_FULL: emf_launch_m<R, TI, TF, TVD_FULL>(c, s); return;
+        case WENO5_FULL: emf_launch_m<R, TI, TF, WENO5_FULL>(c, s); return;
+        case MPWENO5_FULL: emf_launch_m<R, TI, TF, MPWENO5_FULL>(c, s); return;
+        }
+    }
     switch (c->p.reconop) {
     case PDM: emf_launch_m<R, TI, TF, PDM>(c, s); break;
     case TVD: emf_launch_m<R, TI, TF, TVD>(c, s); break;

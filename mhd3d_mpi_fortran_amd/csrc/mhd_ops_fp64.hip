@@ -26,24 +26,16 @@ void launch_recon(mhd_ctx* c, int dir, const double* f, int fn1, int fn2, int ln
     const Coef<double> co = make_coef<double>(c);
     const long n = (long)lnx * lny * lnz;
     const int ng = c->p.ng;
-    switch (c->p.reconop) {
-    case PDM:
-        launch(c, MHD_K_FLUX, blocks(n), dim3(kBlock), k_recon<double, PDM>, ng, dir, f, fn1, fn2, lnx, lny, lnz,
-               co, fl, fr);
-        break;
-    case TVD:
-        launch(c, MHD_K_FLUX, blocks(n), dim3(kBlock), k_recon<double, TVD>, ng, dir, f, fn1, fn2, lnx, lny, lnz,
-               co, fl, fr);
-        break;
-    case WENO5:
-        launch(c, MHD_K_FLUX, blocks(n), dim3(kBlock), k_recon<double, WENO5>, ng, dir, f, fn1, fn2, lnx, lny,
-               lnz, co, fl, fr);
-        break;
-    default:
-        launch(c, MHD_K_FLUX, blocks(n), dim3(kBlock), k_recon<double, MPWENO5>, ng, dir, f, fn1, fn2, lnx, lny,
-               lnz, co, fl, fr);
-        break;
+    auto k = k_recon<double, MPWENO5>;
+    switch (recon_code(c)) {
+    case PDM: k = k_recon<double, PDM>; break;
+    case TVD: k = k_recon<double, TVD>; break;
+    case WENO5: k = k_recon<double, WENO5>; break;
+    case TVD_FULL: k = k_recon<double, TVD_FULL>; break;
+    case WENO5_FULL: k = k_recon<double, WENO5_FULL>; break;
+    case MPWENO5_FULL: k = k_recon<double, MPWENO5_FULL>; break;
     }
+    launch(c, MHD_K_FLUX, blocks(n), dim3(kBlock), k, ng, dir, f, fn1, fn2, lnx, lny, lnz, co, fl, fr);
 }
 
 void launch_vface_fp64(mhd_ctx* c, long n, const double* lam, const double* v, double* v0p, double* v0n, double* v1p,
