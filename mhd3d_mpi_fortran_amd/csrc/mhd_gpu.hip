@@ -132,7 +132,8 @@ int mhd_create(mhd_ctx** out, const mhd_params* p) {
     // index spaces (ghost-inclusive faces and edges) must stay below 2^29, so
     // that every binary64 array stays below 2^32 bytes (32-bit byte offsets
     // in the stencil kernels); about 800^3 cells, which is what the HBM of
-    // one GPU holds for the step's arrays
+    // one GPU holds for the step's arrays (binary64 WENO: with the EMF's scratch,
+    // 18 arrays of 21 planes or up to kWenoScratch, six planes where memory is short)
     if ((double)(p->nx0 + 2 * p->ng + 1) * (p->ny0 + 2 * p->ng + 1) * (p->nz0 + 2 * p->ng + 1) >= 536870912.)
         return MHD_ERR_PARAM;
     for (int a = 0; a < 3; ++a)
@@ -227,19 +228,30 @@ int mhd_create(mhd_ctx** out, const mhd_params* p) {
     }
     size_t total = 0, state = 0;
     for (auto& e : plan) state += e.second;
+    total = state;
     // the EMF's scratch comes last and is not cleared: each launch writes what it reads
-    if ((p->reconop == 3 || p->reconop == 4) && p->precision == MHD_FP64) {
-        const size_t plane = 18 * (size_t)d.nx * d.ny * sizeof(double);
+    const size_t plane = 18 * (size_t)d.nx * d.ny * sizeof(double);
+    const bool weno = (p->reconop == 3 || p->reconop == 4) && p->precision == MHD_FP64;
+    const long fewest = 1 + kWenoHalo;
+    if (weno) {
         const long held = (long)(kWenoScratch / plane);
         const long least = 16 + kWenoHalo, most = d.nz0 + 1 + kWenoHalo;
         c->weno_planes = (int)std::min(most, std::max(least, held));
-        plan.push_back({&c->weno, align_up(plane * c->weno_planes)});
+        if (const char* ev = getenv("MHD_WENO_PLANES")) c->weno_planes = (int)std::min(most, std::max(fewest, atol(ev)));
+        total += align_up(plane * c->weno_planes);
     }
-    for (auto& e : plan) total += e.second;
-    if (hipMalloc(&c->arena, total) != hipSuccess) {
+    bool held = hipMalloc(&c->arena, total) == hipSuccess;
+    if (!held && weno && c->weno_planes > fewest) {
+        (void)hipGetLastError();
+        c->weno_planes = (int)fewest;
+        total = state + align_up(plane * c->weno_planes);
+        held = hipMalloc(&c->arena, total) == hipSuccess;
+    }
+    if (!held) {
         delete c;
         return MHD_ERR_HIP;
     }
+    if (weno) plan.push_back({&c->weno, total - state});
     c->arena_bytes = total;
     size_t off = 0;
     for (auto& e : plan) {

@@ -92,7 +92,9 @@ inline long merge_cells(const mhd_params& p) {
 
 // scratch of the binary64 WENO EMF (mhd_emf_weno.hpp): 18 arrays over a
 // slab of whole planes, as many as kWenoScratch bytes hold (it should stay in
-// the last-level cache), at least kWenoHalo more than 16 planes of edges
+// the last-level cache), at least kWenoHalo more than 16 planes of edges -- or
+// than one, where the GPU's memory does not hold that (environment
+// MHD_WENO_PLANES sets the planes at mhd_create)
 constexpr int kWenoHalo = 5;
 constexpr size_t kWenoScratch = size_t(160) << 20;
 

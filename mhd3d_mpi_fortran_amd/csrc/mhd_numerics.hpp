@@ -39,7 +39,7 @@ struct Coef<double> {
     double wn[3];
     static bool full(double eps) { return !(eps >= 0x1p-400); }
     void set_weno() {
-        const double m = full(eps) ? 1. : std::ldexp(1., std::min(900, 1000 + 2 * std::ilogb(eps)));
+        const double m = full(eps) ? 1. : std::ldexp(1., std::min(900, 1000 + 2 * std::min(0, std::ilogb(eps))));
         wn[0] = .1 * m;
         wn[1] = .6 * m;
         wn[2] = .3 * m;
@@ -66,11 +66,12 @@ __device__ __forceinline__ float qdiv<float>(float a, float b) { return a * __bu
 // instructions instead of 11), so it rounds like it wherever the remainder is
 // representable (|a| above 2^-960; below, the quotient may be one place off).  A
 // smaller divisor gives infinity where a quotient may exist: the limiters' are
-// kept from that by eps (Coef<double>), and gam - 1 is 0 or at least 2^-53.  The
-// flux divides by a pressure as well, which nothing bounds, and has the compiler's
-// division there (256^3 PDM step 5.91 ms, 6.04 with this one; 64^3 TVD 874 us, 864).  The WENO weights' three quotients share one reciprocal (17
-// instructions for 33).  At 96 x 64 x 128 (WENO5) the y flux takes 107 us for 124,
-// the EMF 363 for 443.
+// kept from that by eps (Coef<double>), and gam - 1 is 0 or at least 2^-53 in size.
+// The flux divides by a pressure as well, which nothing bounds, and has the
+// compiler's division there (256^3 PDM step 5.91 ms, 6.04 with this one; five 64^3
+// TVD steps 874 us, 864).  The WENO weights' three quotients share one reciprocal
+// (17 instructions for 33).  At 96 x 64 x 128 (WENO5) the y flux takes 107 us for
+// 124, the EMF 363 for 443.
 template <typename R>
 struct Divisor {
     R b, y;  // y = 1/b
