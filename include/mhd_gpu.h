@@ -274,17 +274,23 @@ void *mhd_device_pointer(mhd_ctx *ctx, int which);
  * kernel classes: see MHD_K_*; *ms = summed duration, *launches = count */
 enum { MHD_K_FLUX = 0, MHD_K_EMF = 1, MHD_K_UPDATE = 2, MHD_K_CT = 3, MHD_K_FILL = 4, MHD_K_BXYZ = 5,
        MHD_K_DT = 6, MHD_K_PREV = 7, MHD_K_SURR = 8, MHD_K_NCLASS = 9 };
-/* (blocks below 2^21 owned cells, binary64 Runge-Kutta ones below 2^25 (TVD
- * 2^22), run a
- * stage's PDM or TVD face fluxes and edge EMFs as one launch, which counts as
- * MHD_K_FLUX; there MHD_K_EMF counts EMFs launched by themselves.  Larger
- * binary64 Adams-Bashforth steps form the z fluxes in the update, which counts
- * as MHD_K_UPDATE, unless the block is narrow along x (PDM then takes the one
- * launch).
+/* A kernel that does the work of several classes counts as one of them:
+ *   - the ghost fill of Runge-Kutta steps and of binary64 or non-periodic
+ *     Adams-Bashforth ones is part of get_bxyz (MHD_K_BXYZ), and the copy of the
+ *     state that a Runge-Kutta step starts from (advance_previous) part of stage
+ *     1's update (MHD_K_UPDATE) and CT (MHD_K_CT);
+ *   - blocks below 2^21 owned cells, binary64 Runge-Kutta ones below 2^25 (TVD
+ *     2^22) and binary64 Adams-Bashforth PDM ones below 2^25 whose rows along x
+ *     fill less than half of their 64-lane tiles run a stage's PDM or TVD face
+ *     fluxes and edge EMFs as one launch, MHD_K_FLUX (MHD_K_EMF: EMFs launched by
+ *     themselves), and its cell update and CT as one, MHD_K_UPDATE;
+ *   - other binary64 Adams-Bashforth steps form the z fluxes in the update,
+ *     MHD_K_UPDATE, where the rows fill 1/2 (PDM), 3/8 (TVD) or 3/4 (WENO5,
+ *     MPWENO5) of their tiles.
  * The learned-reconstruction flux's first pass counts as MHD_K_FLUX;
  * MHD_K_SURR covers its MLP pass over the listed faces, the PDM fallback
  * fix-up, the list reset, sample collection, training and standalone
- * inference) */
+ * inference. */
 int mhd_profile(mhd_ctx *ctx, int enable);
 int mhd_profile_read(mhd_ctx *ctx, int kclass, int *launches, double *ms);
 /* time only the classes whose bit (1 << MHD_K_*) is set in mask (0: off);
@@ -294,12 +300,13 @@ int mhd_profile_read(mhd_ctx *ctx, int kclass, int *launches, double *ms);
 int mhd_profile_classes(mhd_ctx *ctx, unsigned mask);
 
 /* stage scheduling (no counterpart in the reference): on (the default for
- * blocks of at least 2^21 owned cells, binary64 Runge-Kutta ones of at
- * least 2^25, 2^22 with TVD), a stage's edge EMF and CT run on a
- * second stream beside its face flux and cell update; off (the default for
- * smaller blocks, and for ensemble members), every kernel runs on the
- * context's stream in the reference's order (the per-kernel times then add
- * up to the step).  The results are the same bit for bit either way. */
+ * blocks of at least 2^21 owned cells, except the larger ones listed at
+ * mhd_profile that run a stage's stencils as one launch), a stage's edge EMF and
+ * CT run on a second stream beside its face flux and cell update; off (the
+ * default for the others, and for ensemble members), every kernel runs on the
+ * context's stream, in the reference's order up to the launches that the list at
+ * mhd_profile combines (the per-kernel times then add up to the step).  The
+ * results are the same bit for bit either way. */
 int mhd_set_stage_overlap(mhd_ctx *ctx, int on);
 
 /* kernel fusion (no counterpart in the reference): on, a mixed-precision

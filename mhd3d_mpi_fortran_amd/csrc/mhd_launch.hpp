@@ -139,7 +139,9 @@ struct mhd_ctx {
     long ndt_valid = 0;      // ... that many of them
     bool spacing_mid = false;  // the update's spacings lie within 2^-400 .. 2^400
     bool ghost_twins = false;  // every ghost cell repeats an owned cell (periodic axes, equal ghost spacings)
-    bool cellb_stale = false;  // bx,by,bz not stored for the current state (mixed AB steps, uploads, advances)
+    // bx,by,bz not stored for the current state (mixed AB steps, all but a call's
+    // last stage of mixed RK ones, uploads, advances)
+    bool cellb_stale = false;
     bool pred_valid = false;   // the extrapolated state of mhd_predict_ab is held (xh / fp32 copies)
     // per-stage products (binary64, or fp32 in mixed precision)
     void* flux[3] = {nullptr, nullptr, nullptr};

@@ -68,8 +68,8 @@ __device__ __forceinline__ float qdiv<float>(float a, float b) { return a * __bu
 // smaller divisor gives infinity where a quotient may exist: the limiters' are
 // kept from that by eps (Coef<double>), and gam - 1 is 0 or at least 2^-53 in size.
 // The flux divides by a pressure as well, which nothing bounds, and has the
-// compiler's division there (256^3 PDM step 5.91 ms, 6.04 with this one; five 64^3
-// TVD steps 874 us, 864).  The WENO weights' three quotients share one reciprocal
+// compiler's division there (256^3 PDM step 6.07 ms, 6.06 with this one; five 64^3
+// PDM steps 931 us, 925, TVD 850 and 842).  The WENO weights' three quotients share one reciprocal
 // (17 instructions for 33).  At 96 x 64 x 128 (WENO5) the y flux takes 107 us for
 // 124, the EMF 363 for 443.
 template <typename R>

@@ -32,8 +32,9 @@ struct EmfSteps {
 // take several times what their arithmetic needs.  The grid is the six
 // kernels' workgroups end to end, the EMF's (the longest) first; every
 // workgroup belongs to one of them.  Its registers are the largest of the six,
-// which large blocks would pay for in the flux: they keep the separate
-// kernels, EMF and flux on two streams.  A stage of 64^3 (PDM, binary64) took
+// which large blocks would pay for in the flux: blocks past the size to which the
+// one launch measured faster (merge_cells) keep the separate kernels, EMF and flux
+// on two streams.  A stage of 64^3 (PDM, binary64) took
 // 114 us with the six kernels and takes 84 us, 16^3 51 and 12 us.
 template <typename R, typename TF>
 struct StencilOut {

@@ -116,7 +116,7 @@ __global__ void __launch_bounds__(kBlock) k_ct(Dims d, const double* __restrict_
 
 // Blocks whose stage runs in one stream (k_stencils): the cell update and CT,
 // which are independent, in one launch -- the update's workgroups, then CT's.
-// Large blocks keep the two kernels, CT beside the flux.  (met: the metric's
+// Blocks past that (merge_cells) keep the two kernels, CT beside the flux.  (met: the metric's
 // spacing for the update; CT takes the computational one.)  16^3: 8.4 us for
 // the two kernels, 4.6 for this; 64^3: 24 and 21 us.
 template <int NST, int ST, typename TF, bool GEN>
@@ -332,7 +332,7 @@ __global__ void __launch_bounds__(kBlock) k_bxyz(Dims d, double gam, double cfl,
                 if (met.ws[a]) met.ws[a][t] = float(wn);
             }
         }
-        if (bx) {  // null: the caller keeps cell B implicit (mixed Adams-Bashforth)
+        if (bx) {  // null: the caller keeps cell B implicit (mixed steps)
             bx[t] = x;
             by[t] = y;
             bz[t] = z;

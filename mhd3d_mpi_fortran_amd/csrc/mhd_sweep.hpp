@@ -17,11 +17,12 @@ namespace mhd {
 // The z products need not be read back, nor, but for a call's last step, be
 // written (128 bytes a cell), and the update's loads run beside other wavefronts'
 // flux arithmetic: at 256^3 (PDM) z flux and update take 1.51 ms for 0.87 + 0.94,
-// the step 5.87 ms for 6.21; 128^3 859 us for 901, 33 x 400 x 160 1187 for 1206,
-// 1000 x 600 x 5 1.68 ms for 1.79; TVD 192^3 2.29 ms for 2.45, WENO5 and MPWENO5
-// 128^3 1 to 2 % less.  Bound by latency at 3 wavefronts a SIMD (168 VGPRs; capped
-// at 128 it took 1.74 ms, and with the x and y differences loaded before the
-// flux 1.80).  The same in binary32 took 1.48 ms for 0.26 + 0.68 and is not here.
+// the step 5.87 ms for 6.21; 128^3 859 us for 901, 1000 x 600 x 5 1.68 ms for 1.79
+// (rows that leave lanes idle: sweep_fills); TVD 192^3 2.29 ms for 2.45, WENO5 and
+// MPWENO5 128^3 1 to 2 % less.  Bound by memory traffic, 8.1 GB (compulsory 4.6) at the
+// 5.3 TB/s that a copy reaches, with 3 wavefronts a SIMD (168 VGPRs; capped at 128
+// it took 1.74 ms, and with the x and y differences loaded before the flux 1.80).
+// The same in binary32 took 1.48 ms for 0.26 + 0.68 and is not here.
 template <int M, int MET>
 __global__ void __launch_bounds__(kBlock)
     k_sweep_update(Dims d, Coef<double> c, Prim<double> q, Normals<double> nm, SweepArgs a) {
